@@ -72,7 +72,10 @@ const char *ternocl_version(void);
  * Replaces int2_fp16_upcvt_gemm (decode, int2_fp16_upcvt/int2_fp16_upcvt.cl:196-198)
  * and int2_fp16_upcvt_gemm_mt (prefill, :341-343):
  *   C[m,n] = ct(epi(sum_g S[g,n] * sum_{k in g} A[m,k] * code(B[k,n])))
- * The library picks the kernel: a decode GEMV for M <= 16, an MFMA GEMM above.
+ * The library picks the kernel: a decode GEMV for M <= 8, an MFMA GEMM that
+ * splits K over the waves of a workgroup for M from 9 to several hundred
+ * (operands 16-byte aligned; the MFMA GEMV / the tile GEMM otherwise), an MFMA
+ * tile GEMM above.
  * ws / ws_bytes: optional device scratch (16-byte aligned), kept from the XeTLA
  * plugin's entry (the acc/cnt buffers of its global k-slicing,
  * tools/xetla_epilogue_parity/parity.cpp:26-41); ternocl_int2_gemm_ws_bytes()

@@ -67,6 +67,13 @@ ternocl_status int2_gemm_mfma_run(int dtype, const void *A, const uint32_t *B, c
                                   size_t ws_bytes = 0);
 size_t int2_gemm_ws_need(int M, int N, int K);
 ternocl_status int2_gemm_decode_run(int dtype, const uint32_t *B, uint32_t *D, int K, int N, hipStream_t st);
+// kernels (int2_gemm_kw.hip)
+bool int2_gemm_kw_auto(int M, int N, int K, bool split, const void *A, const void *B, const void *S, const void *C,
+                       const void *Other, const void *Bias);
+size_t int2_gemm_kw_ws_need(int M, int N, int K);
+ternocl_status int2_gemm_kw_run(int dtype, const void *A, const uint32_t *B, const void *S, void *C, const void *Other,
+                                const void *Bias, int M, int N, int K, int postop, int out_f32, hipStream_t st,
+                                bool split, void *ws);
 // kernels (int2_int8.hip)
 ternocl_status quant_a_run(int dtype, const void *A, void *SA, int8_t *Aq, int M, int K, hipStream_t st,
                            const int *perm = nullptr, int topk = 1, const int *nrows = nullptr);
@@ -189,8 +196,9 @@ size_t ternocl_int2_gemm_ws_bytes(int M, int N, int K) {
     if (M < 1 || N < 16 || N % 16 || K < kGS || K % kGS) return 0;
     // the fp8 x fp4 GEMV's K split: slice sums and a counter per strip
     if (M <= 16) return int2_gemv_f4_ws_need(M, N, K);
-    // the prefill GEMM's split-K partials (shapes whose 128 x 512 tiles leave CUs idle)
-    return int2_gemm_ws_need(M, N, K);
+    // the slice sums of the K-split engines' plans (an upper bound of the two)
+    const size_t a = int2_gemm_ws_need(M, N, K), b = int2_gemm_kw_ws_need(M, N, K);
+    return a > b ? a : b;
 }
 
 ternocl_status ternocl_workspace_zero(void *ws, size_t ws_bytes, void *stream) {
@@ -208,19 +216,24 @@ ternocl_status ternocl_int2_fp16_upcvt_gemm_ex(int dtype, const void *A, const u
     const ternocl_gemv_tile t = tile ? *tile : ternocl_gemv_tile{0, 0, 0, 0, 0, 0};
     if (t.engine < 0 || t.engine > 5) FAIL(TERNOCL_ERR_INVALID_ARG, "tile engine must be 0..5");
     if (t.k_slices < 0 || t.k_slices > 16) FAIL(TERNOCL_ERR_INVALID_ARG, "k_slices must be 0..16");
+    const bool auto_tile = t.engine == 0 && t.waves == 0 && t.cols_per_lane == 0 && t.groups_per_wave == 0 && t.k_slices == 0;
     if (t.engine == 3 || (M > 16 && t.engine == 0)) {
         if (t.k_slices > 1) FAIL(TERNOCL_ERR_INVALID_ARG, "k_slices > 1: the fp8 x fp4 GEMV (engine 4) only");
         // the GEMM addresses the packed weights with 32-bit buffer offsets
         if ((size_t)(K / 16) * (size_t)N * 4 >= kMaxBufBytes)
             FAIL(TERNOCL_ERR_UNSUPPORTED_SHAPE, "the prefill GEMM takes packed weights (K * N / 4 bytes) below 2^31 bytes");
+        // automatic: K split over the waves where that model is ahead (tens to hundreds of rows)
+        const size_t need = int2_gemm_kw_ws_need(M, N, K);
+        const bool split = need && ws && ws_bytes >= need && ((uintptr_t)ws & 15) == 0;
+        if (t.engine == 0 && int2_gemm_kw_auto(M, N, K, split, A, B, S, C, Other, Bias))
+            return int2_gemm_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream, split, ws);
         return int2_gemm_mfma_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32,
                                   (hipStream_t)stream, ws, ws_bytes);
     }
     if (M <= 16) {
         // automatic: the fp8 x fp4 engine where it applies (its multi-strip
-        // kernel on many strips), else the bf16/fp16 MFMA GEMV
-        const bool auto_tile = t.engine == 0 && t.waves == 0 && t.cols_per_lane == 0 && t.groups_per_wave == 0 &&
-                               t.k_slices == 0;
+        // kernel on many strips), else the GEMM with K split over the waves
+        // (9..16 rows), else (unaligned operands) the bf16/fp16 MFMA GEMV
         if (t.engine == 5 || (auto_tile && int2_gemv_f4_supports(M, N, A) && int2_gemv_f4ms_auto(M, N, K))) {
             if (t.waves)
                 FAIL(TERNOCL_ERR_INVALID_ARG, "the multi-strip GEMV (engine 5) takes cols_per_lane, "
@@ -240,6 +253,8 @@ ternocl_status ternocl_int2_fp16_upcvt_gemm_ex(int dtype, const void *A, const u
             return int2_gemv_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, t.waves,
                                  t.col_lanes, (hipStream_t)stream);
         }
+        if (auto_tile && int2_gemm_kw_auto(M, N, K, false, A, B, S, C, Other, Bias))
+            return int2_gemm_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream, false, nullptr);
         return int2_gemv_mfma_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, t.waves,
                                   t.cols_per_lane, t.groups_per_wave, (hipStream_t)stream);
     }
