@@ -198,8 +198,10 @@ ternocl_status ternocl_quant_a(int dtype, const void *A, void *SA, int8_t *Aq, i
  * ternocl_int2_fp16_upcvt_gemm.  Any M >= 1; the A operand (M*K elements of
  * Aq or A) and B must each be below 2^31 bytes.  M <= 4 with N % 16 == 0 (Aq
  * 8-byte or A 16-byte aligned) runs the decode GEMV (the reference's
- * int2_int8_gemv): the same exact group dot products and the same fold, with
- * the groups of a column summed in a different order than the tile GEMM. */
+ * int2_int8_gemv), and M from 5 to several hundred (operands 16-byte aligned) a
+ * GEMM that splits K over the waves of a workgroup: the same exact group dot
+ * products and the same fold, with the groups of a column summed in a different
+ * order than the tile GEMM. */
 ternocl_status ternocl_int2_int8_gemm(int dtype, const void *A, const int8_t *Aq, const void *SA,
                                       const uint32_t *B, const void *SB, void *C,
                                       const void *Other, const void *Bias, int M, int N, int K,

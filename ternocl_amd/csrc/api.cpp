@@ -82,6 +82,7 @@ ternocl_status int2_int8_gemm_run(int dtype, const void *A, const int8_t *Aq, co
                                   const void *Bias, int M, int N, int K, int postop, int out_f32,
                                   hipStream_t st, void *ws = nullptr, size_t ws_bytes = 0);
 ternocl_status int2_s8_decode_run(const uint32_t *B, uint32_t *D, int K, int N, hipStream_t st);
+size_t int2_int8_kw_ws_need(int M, int N, int K);  // int2_int8_kw.hip
 // kernels (bitcos.hip)
 int bitcos_max_ls();
 int bitcos_pick_ls(int N, int K);
@@ -345,7 +346,9 @@ ternocl_status ternocl_int2_int8_gemm(int dtype, const void *A, const int8_t *Aq
 size_t ternocl_int2_int8_gemm_ws_bytes(int M, int N, int K) {
     if (M < 1 || N < 16 || N % 16 || K < kGS || K % kGS) return 0;
     if (M <= 4) return int2_int8_gemv_ws_need(M, N, K);  // the decode GEMV's K split
-    return int2_gemm_ws_need(M, N, K);
+    // the slice sums of the K-split engines' plans (an upper bound of the two)
+    const size_t a = int2_gemm_ws_need(M, N, K), b = int2_int8_kw_ws_need(M, N, K);
+    return a > b ? a : b;
 }
 
 ternocl_status ternocl_int2_s8_decode(const uint32_t *B, uint32_t *D, int K, int N, void *stream) {

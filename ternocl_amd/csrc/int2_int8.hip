@@ -36,7 +36,7 @@
 //     the order of the reference's host gold (int2_via_int2_x_int8_dpas/main.cpp:113-116);
 //     the fold of block mb runs between the MFMAs of block mb + 1;
 //   * all loads are buffer loads with offsets computed once per kernel.
-#include "common.hpp"
+#include "int8_frag.hpp"
 
 #include <cfloat>
 
@@ -45,16 +45,21 @@ namespace tcl {
 // and its rule for 128 x 256 tiles)
 int gemm_splits(int M, int N, int K);
 bool gemm_half_tile(int M, int N);
+// (int2_int8_kw.hip)
+bool int2_int8_kw_auto(int M, int N, int K, bool split, const void *A, const void *B, const void *SB, const void *C,
+                       const void *Other, const void *Bias);
+size_t int2_int8_kw_ws_need(int M, int N, int K);
+hipError_t int2_int8_kw_run(int dtype, const void *A, const int8_t *Aq, const void *SA, const uint32_t *B, const void *SB,
+                            void *C, const void *Other, const void *Bias, int M, int N, int K, int postop, int out_f32,
+                            hipStream_t st, bool split, void *ws);
 hipError_t splitk_reduce_launch(int dtype, const float *part, int splits, void *C, const void *Other,
                                 const void *Bias, int M, int N, int postop, int out_f32, hipStream_t st);
 namespace {
 
-typedef int i32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr float kEps = FLT_EPSILON;  // xetla's absmax floor, int2_int8_dpas.cl:59
 
-__host__ __device__ constexpr int ldsa_of(int M) { return (M + 31) & ~31; }
 
 // ---- quant_a ---------------------------------------------------------------
 
@@ -103,29 +108,6 @@ k_quant_a(const uint16_t *__restrict__ A, uint16_t *__restrict__ SA, int8_t *__r
 // ---- s8 x s2 GEMM ------------------------------------------------------------
 
 constexpr int QA_PITCH = 144;  // bytes per LDS row of the A tile (128 + 16: conflict-free b128 reads)
-constexpr uint32_t kCodeLut = 0xFFFE0100u;  // int8 of code 0, 1, 2, 3
-
-// out[i] byte b = byte i of d[b] (4 x 4 byte transpose)
-__device__ __forceinline__ void transpose4x4(const uint32_t d[4], uint32_t o[4]) {
-    const uint32_t p0 = __builtin_amdgcn_perm(d[1], d[0], 0x06020400u);  // d0.b0 d1.b0 d0.b2 d1.b2
-    const uint32_t p1 = __builtin_amdgcn_perm(d[1], d[0], 0x07030501u);  // d0.b1 d1.b1 d0.b3 d1.b3
-    const uint32_t p2 = __builtin_amdgcn_perm(d[3], d[2], 0x06020400u);
-    const uint32_t p3 = __builtin_amdgcn_perm(d[3], d[2], 0x07030501u);
-    o[0] = __builtin_amdgcn_perm(p2, p0, 0x05040100u);
-    o[1] = __builtin_amdgcn_perm(p3, p1, 0x05040100u);
-    o[2] = __builtin_amdgcn_perm(p2, p0, 0x07060302u);
-    o[3] = __builtin_amdgcn_perm(p3, p1, 0x07060302u);
-}
-
-// B fragment of one word: dword i byte b = int8 value of row 4b + i.
-__device__ __forceinline__ i32x4_t decode_s2(uint32_t w) {
-    i32x4_t r;
-    r[0] = (int)__builtin_amdgcn_perm(kCodeLut, kCodeLut, w & 0x03030303u);
-    r[1] = (int)__builtin_amdgcn_perm(kCodeLut, kCodeLut, (w >> 2) & 0x03030303u);
-    r[2] = (int)__builtin_amdgcn_perm(kCodeLut, kCodeLut, (w >> 4) & 0x03030303u);
-    r[3] = (int)__builtin_amdgcn_perm(kCodeLut, kCodeLut, (w >> 6) & 0x03030303u);
-    return r;
-}
 
 // Tile shape: WVM x WVN waves, each owning MB x CB blocks of 16 x 16 outputs.
 template <int MB_, int CB_, int WVM_, int WVN_> struct QTile {
@@ -145,16 +127,6 @@ template <int MB_, int CB_, int WVM_, int WVN_> struct QTile {
 template <int CB> struct QBSlab {
     uint32_t w[CB][2], sb[CB];
 };
-
-// In-GEMM quantization (the reference's QMODE 1, int2_int8_dpas.cl:61-68 and
-// quant8x32 :70-99): the int8 of a DT activation is the low byte of
-// fma(a, sa, 1.5 * 2^23), which rounds a * sa (exact in fp32) to the nearest
-// even integer; |a * sa| <= 127.06 by the construction of sa, so it equals
-// quant_a's saturating conversion for every finite input.
-template <bool BF16>
-__device__ __forceinline__ uint32_t q8_bits(uint32_t h, float sa) {
-    return __float_as_uint(__builtin_fmaf(dt2f<BF16>(h), sa, 12582912.0f));
-}
 
 // QA = false: A tiles come from Aq (int8, written by quant_a: the reference's
 // QMODE 0).  QA = true: from the DT activations A, quantized while staged.
@@ -873,6 +845,11 @@ ternocl_status int2_int8_gemm_run(int dtype, const void *A, const int8_t *Aq, co
         set_error("int2_int8_gemm: the A operand and B must each be below 2^31 bytes");
         return TERNOCL_ERR_UNSUPPORTED_SHAPE;
     }
+    // few to hundreds of rows: K split over the waves where that model is ahead
+    const size_t kw_need = int2_int8_kw_ws_need(M, N, K);
+    const bool kw_split = kw_need && ws && ((uintptr_t)ws & 15) == 0 && ws_bytes >= kw_need;
+    if (int2_int8_kw_auto(M, N, K, kw_split, Aq ? (const void *)Aq : A, B, SB, C, Other, Bias))
+        return launch_status(int2_int8_kw_run(dtype, A, Aq, SA, B, SB, C, Other, Bias, M, N, K, postop, out_f32, st, kw_split, ws));
     // 128 x 256 tiles of eight 128 x 32 waves where 128 x 128 tiles would
     // number more than 256 and 128 x 256 tiles fit one per CU (the fp16
     // prefill GEMM's rule): they decode each weight word for 128 rows, the
