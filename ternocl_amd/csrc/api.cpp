@@ -68,7 +68,7 @@ ternocl_status int2_gemm_mfma_run(int dtype, const void *A, const uint32_t *B, c
 size_t int2_gemm_ws_need(int M, int N, int K);
 ternocl_status int2_gemm_decode_run(int dtype, const uint32_t *B, uint32_t *D, int K, int N, hipStream_t st);
 // kernels (int2_gemm_kw.hip)
-bool int2_gemm_kw_auto(int M, int N, int K, bool split, const void *A, const void *B, const void *S, const void *C,
+bool int2_gemm_kw_auto(int M, int N, int K, bool split, bool bf, const void *A, const void *B, const void *S, const void *C,
                        const void *Other, const void *Bias);
 size_t int2_gemm_kw_ws_need(int M, int N, int K);
 ternocl_status int2_gemm_kw_run(int dtype, const void *A, const uint32_t *B, const void *S, void *C, const void *Other,
@@ -94,6 +94,11 @@ size_t bitcos_gemv_ws_need(int N, int ls);
 ternocl_status bitcos_gemm_mt_run(int dtype, const void *A, const uint32_t *Bc, const void *S, void *C,
                                   const void *Other, const void *Bias, int M, int N, int K, int postop,
                                   int out_f32, hipStream_t st);
+// kernels (bitcos_kw.hip): how a call of the M-tiled entry runs there (0: not)
+int bitcos_kw_auto(int M, int N, int K, bool bf, bool repack, const void *A, const void *Bc, const void *S, const void *C,
+                   const void *Other, const void *Bias);
+ternocl_status bitcos_kw_run(int dtype, const void *A, const uint32_t *Bc, const void *S, void *C, const void *Other,
+                             const void *Bias, int M, int N, int K, int postop, int out_f32, hipStream_t st);
 ternocl_status bitcos_slice_ranks_run(const uint32_t *Bc, uint32_t *SR, int N, int K, int ls,
                                       hipStream_t st);
 ternocl_status bitcos_dequant_run(int dtype, const uint32_t *Bc, const void *S, void *W, int N, int K,
@@ -226,7 +231,7 @@ ternocl_status ternocl_int2_fp16_upcvt_gemm_ex(int dtype, const void *A, const u
         // automatic: K split over the waves where that model is ahead (tens to hundreds of rows)
         const size_t need = int2_gemm_kw_ws_need(M, N, K);
         const bool split = need && ws && ws_bytes >= need && ((uintptr_t)ws & 15) == 0;
-        if (t.engine == 0 && int2_gemm_kw_auto(M, N, K, split, A, B, S, C, Other, Bias))
+        if (t.engine == 0 && int2_gemm_kw_auto(M, N, K, split, dtype == TERNOCL_BF16, A, B, S, C, Other, Bias))
             return int2_gemm_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream, split, ws);
         return int2_gemm_mfma_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32,
                                   (hipStream_t)stream, ws, ws_bytes);
@@ -254,7 +259,7 @@ ternocl_status ternocl_int2_fp16_upcvt_gemm_ex(int dtype, const void *A, const u
             return int2_gemv_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, t.waves,
                                  t.col_lanes, (hipStream_t)stream);
         }
-        if (auto_tile && int2_gemm_kw_auto(M, N, K, false, A, B, S, C, Other, Bias))
+        if (auto_tile && int2_gemm_kw_auto(M, N, K, false, dtype == TERNOCL_BF16, A, B, S, C, Other, Bias))
             return int2_gemm_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream, false, nullptr);
         return int2_gemv_mfma_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, t.waves,
                                   t.cols_per_lane, t.groups_per_wave, (hipStream_t)stream);
@@ -438,6 +443,8 @@ ternocl_status ternocl_bitcos_fp16_upcvt_gemm_mt(int dtype, const void *A, const
     if (!ws) {  // the tiles decode the BITCOS weights themselves
         if ((size_t)M * K * 2 >= kMaxBufBytes)
             FAIL(TERNOCL_ERR_UNSUPPORTED_SHAPE, "the M-tiled BITCOS GEMM takes A below 2^31 bytes");
+        if (bitcos_kw_auto(M, N, K, dtype == TERNOCL_BF16, false, A, B, S, C, Other, Bias))
+            return bitcos_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream);
         return bitcos_gemm_mt_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream);
     }
     const size_t need = ternocl_bitcos_gemm_mt_ws_bytes(K, N);
@@ -447,7 +454,11 @@ ternocl_status ternocl_bitcos_fp16_upcvt_gemm_mt(int dtype, const void *A, const
         FAIL(TERNOCL_ERR_UNSUPPORTED_SHAPE, "the M-tiled BITCOS path takes A and the re-packed weights below 2^31 bytes");
     const hipStream_t st = (hipStream_t)stream;
     uint32_t *W2 = (uint32_t *)((uint8_t *)ws + kWsHeader);
+    const int kw = bitcos_kw_auto(M, N, K, dtype == TERNOCL_BF16, true, A, B, S, C, Other, Bias);
+    if (kw == 1) return bitcos_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, st);
     if ((s = bitcos_to_int2_run(B, SR, ls, W2, N, K, st)) != TERNOCL_OK) return s;
+    if (kw == 2)
+        return int2_gemm_kw_run(dtype, A, W2, S, C, Other, Bias, M, N, K, postop, out_f32, st, false, nullptr);
     return int2_gemm_mfma_run(dtype, A, W2, S, C, Other, Bias, M, N, K, postop, out_f32, st);
 }
 

@@ -83,6 +83,14 @@ template <int CB, int PF> struct KwInt2 {
         bw[s][1] = __builtin_nontemporal_load((const W *)(p + vb1));
         sr[s] = *(const SV *)(S + (size_t)(uc >> 1) * N + col);
     }
+    __device__ __forceinline__ void start(int u0) {
+#pragma unroll
+        for (int s = 0; s < PF; ++s) load(u0 + s, s);
+    }
+    // unit u's words are taken from slot s: refill it (more: a unit u + PF may follow)
+    __device__ __forceinline__ void next(int u, int s, bool more) {
+        if (more) load(u + PF, s);
+    }
     // slot s's words and each column's scale byte tables {0, s, 0, -s}
     __device__ __forceinline__ void get(int s, uint32_t w[CB][2], uint32_t lo[CB], uint32_t hi[CB]) {
         uint32_t sw[(CB + 1) / 2] = {}, t0[CB], t1[CB];
@@ -134,7 +142,7 @@ __device__ __forceinline__ void kw_walk(uint8_t *abuf, const uint16_t *A, const 
         const int p = s & 1;
         uint32_t w[CB][2], lo[CB], hi[CB];
         bs.get(s, w, lo, hi);
-        if (more) bs.load(u + PF, s);
+        bs.next(u, s, more);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {  // MFMA k-steps: word t = i / 2, half h = i % 2
@@ -163,8 +171,7 @@ __device__ __forceinline__ void kw_walk(uint8_t *abuf, const uint16_t *A, const 
     };
     if (u0 < u1) {
         a_load(u0);
-#pragma unroll
-        for (int s = 0; s < PF; ++s) bs.load(u0 + s, s);
+        bs.start(u0);
         __builtin_amdgcn_sched_barrier(0);
         a_store(0);
         a_load(u0 + 1);

@@ -140,18 +140,19 @@ KwPlan kw_plan(int M, int N, int K, bool split) {
 
 // The 128-row tile engine's time (int2_gemm_mfma.hip) by the same kind of fit, over its
 // plan: 128 x 128 tiles (M = 32 / 512 / 1024, K = N = 4096: 39.8 / 43.5 / 48.9
-// us), 128 x 256 tiles (M = 1024, K = 4096, N = 6144: 66.7; M = 194, K = 13184, N =
-// 23936: 183), 128 x 512 tiles (N = 14336: 103) and their K split.  Both fits are
+// us), 128 x 256 tiles, dearer in bf16 (M = 300, K = 4096, N = 14336: 67.1; fp16 M = 194,
+// K = 13184, N = 23936: 183, M = 64, K = 5376, N = 21504: 53), 128 x 512 tiles (N =
+// 14336: 103) and their K split.  Both fits are
 // good to some 5%, so this engine is taken where it is ahead by more (kKwMargin).
 constexpr double kKwMargin = 0.95;
-double kw_other_us(int M, int N, int K, bool split) {
+double kw_other_us(int M, int N, int K, bool split, bool bf) {
     auto tiles = [&](int BM, int BN) { return (double)((long)((M + BM - 1) / BM) * ((N + BN - 1) / BN)); };
     const double k = K / 1024.0, wide = tiles(128, 512), half = tiles(128, 256), square = tiles(128, 128);
     if (wide >= 192) return 5.0 + 24.5 * k * (wide <= 256 ? 1.0 : wide / 256.0);
     const bool h = gemm_half_tile(M, N);
     const int ks = split && !(h && half >= 192) ? gemm_splits(M, N, K) : 1;
     if (ks > 1) return 8.0 + 24.5 * k / ks + 8e-6 * ks * M * N / 4.0;
-    if (h) return 8.0 + 13.8 * k;
+    if (h) return 5.0 + (6.4 + 9.0 * half / 256.0 + (bf ? 3.0 : 0.0)) * k;
     if (square <= 512) return 3.2 + (9.3 + 1.8 * std::min(square, 256.0) / 256.0) * k * (square > 256 ? 1.5 : 1.0);
     return 5.0 + 24.5 * k * (wide <= 256 ? 1.0 : wide / 256.0);
 }
@@ -160,23 +161,34 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
 
+// The times the two models give a call without a K split (the M-tiled BITCOS
+// GEMM's choice, bitcos_kw.hip); wk: the waves over K of this engine's tile.
+void int2_gemm_kw_model(int M, int N, int K, bool bf, double &kw_us, double &other_us, int &wk) {
+    const KwPlan p = kw_plan(M, N, K, false);
+    kw_us = p.us;
+    other_us = kw_other_us(M, N, K, false, bf);
+    wk = p.tile <= 1 ? 8 : 4;
+}
+
 // Whether the automatic engine of a call of M > 8 rows is this one: always up
 // to 16 rows (the MFMA GEMV is 2-3x its time there), above where its model is
 // ahead of the 128-row tile engine's.  split: whether K slices may use a
-// workspace.  The vector loads and stores need 16-byte aligned operands.
-bool int2_gemm_kw_auto(int M, int N, int K, bool split, const void *A, const void *B, const void *S, const void *C,
+// workspace.
+static bool kw_wins(int M, int N, int K, bool split, bool bf) {
+    return M <= 16 || (M <= 2048 && kw_plan(M, N, K, split).us < kKwMargin * kw_other_us(M, N, K, split, bf));
+}
+// (the vector loads and stores need 16-byte aligned operands)
+bool int2_gemm_kw_auto(int M, int N, int K, bool split, bool bf, const void *A, const void *B, const void *S, const void *C,
                        const void *Other, const void *Bias) {
-    if (M <= 8 || !aligned16(A) || !aligned16(B) || !aligned16(S) || !aligned16(C) || !aligned16(Other) || !aligned16(Bias))
-        return false;
-    if (M <= 16) return true;
-    return M <= 2048 && kw_plan(M, N, K, split).us < kKwMargin * kw_other_us(M, N, K, split);
+    return M > 8 && aligned16(A) && aligned16(B) && aligned16(S) && aligned16(C) && aligned16(Other) && aligned16(Bias) &&
+           kw_wins(M, N, K, split, bf);
 }
 
 // Workspace of the automatic plan's K split (0: none; none up to 16 rows).
 size_t int2_gemm_kw_ws_need(int M, int N, int K) {
     if (M <= 16 || M > 2048) return 0;
     const KwPlan p = kw_plan(M, N, K, true);
-    return p.ks > 1 && p.us < kKwMargin * kw_other_us(M, N, K, true) ? kWsHeader + (size_t)p.ks * M * N * 4 : 0;
+    return p.ks > 1 && (kw_wins(M, N, K, true, false) || kw_wins(M, N, K, true, true)) ? kWsHeader + (size_t)p.ks * M * N * 4 : 0;
 }
 
 // split: K slices may use ws (int2_gemm_kw_ws_need bytes, 16-byte aligned).
