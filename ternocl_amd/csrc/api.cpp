@@ -68,12 +68,10 @@ ternocl_status int2_gemm_mfma_run(int dtype, const void *A, const uint32_t *B, c
 size_t int2_gemm_ws_need(int M, int N, int K);
 ternocl_status int2_gemm_decode_run(int dtype, const uint32_t *B, uint32_t *D, int K, int N, hipStream_t st);
 // kernels (int2_gemm_kw.hip)
-bool int2_gemm_kw_auto(int M, int N, int K, bool split, bool bf, const void *A, const void *B, const void *S, const void *C,
-                       const void *Other, const void *Bias);
 size_t int2_gemm_kw_ws_need(int M, int N, int K);
-ternocl_status int2_gemm_kw_run(int dtype, const void *A, const uint32_t *B, const void *S, void *C, const void *Other,
-                                const void *Bias, int M, int N, int K, int postop, int out_f32, hipStream_t st,
-                                bool split, void *ws);
+bool int2_gemm_kw_run(int dtype, const void *A, const uint32_t *B, const void *S, void *C, const void *Other,
+                      const void *Bias, int M, int N, int K, int postop, int out_f32, hipStream_t st, void *ws,
+                      size_t ws_bytes, bool force, ternocl_status &s);
 // kernels (int2_int8.hip)
 ternocl_status quant_a_run(int dtype, const void *A, void *SA, int8_t *Aq, int M, int K, hipStream_t st,
                            const int *perm = nullptr, int topk = 1, const int *nrows = nullptr);
@@ -229,10 +227,9 @@ ternocl_status ternocl_int2_fp16_upcvt_gemm_ex(int dtype, const void *A, const u
         if ((size_t)(K / 16) * (size_t)N * 4 >= kMaxBufBytes)
             FAIL(TERNOCL_ERR_UNSUPPORTED_SHAPE, "the prefill GEMM takes packed weights (K * N / 4 bytes) below 2^31 bytes");
         // automatic: K split over the waves where that model is ahead (tens to hundreds of rows)
-        const size_t need = int2_gemm_kw_ws_need(M, N, K);
-        const bool split = need && ws && ws_bytes >= need && ((uintptr_t)ws & 15) == 0;
-        if (t.engine == 0 && int2_gemm_kw_auto(M, N, K, split, dtype == TERNOCL_BF16, A, B, S, C, Other, Bias))
-            return int2_gemm_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream, split, ws);
+        if (t.engine == 0 && int2_gemm_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream,
+                                              ws, ws_bytes, false, s))
+            return s;
         return int2_gemm_mfma_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32,
                                   (hipStream_t)stream, ws, ws_bytes);
     }
@@ -259,8 +256,9 @@ ternocl_status ternocl_int2_fp16_upcvt_gemm_ex(int dtype, const void *A, const u
             return int2_gemv_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, t.waves,
                                  t.col_lanes, (hipStream_t)stream);
         }
-        if (auto_tile && int2_gemm_kw_auto(M, N, K, false, dtype == TERNOCL_BF16, A, B, S, C, Other, Bias))
-            return int2_gemm_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream, false, nullptr);
+        if (auto_tile && int2_gemm_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream,
+                                          nullptr, 0, false, s))
+            return s;
         return int2_gemv_mfma_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, t.waves,
                                   t.cols_per_lane, t.groups_per_wave, (hipStream_t)stream);
     }
@@ -457,8 +455,8 @@ ternocl_status ternocl_bitcos_fp16_upcvt_gemm_mt(int dtype, const void *A, const
     const int kw = bitcos_kw_auto(M, N, K, dtype == TERNOCL_BF16, true, A, B, S, C, Other, Bias);
     if (kw == 1) return bitcos_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, st);
     if ((s = bitcos_to_int2_run(B, SR, ls, W2, N, K, st)) != TERNOCL_OK) return s;
-    if (kw == 2)
-        return int2_gemm_kw_run(dtype, A, W2, S, C, Other, Bias, M, N, K, postop, out_f32, st, false, nullptr);
+    if (kw == 2 && int2_gemm_kw_run(dtype, A, W2, S, C, Other, Bias, M, N, K, postop, out_f32, st, nullptr, 0, true, s))
+        return s;
     return int2_gemm_mfma_run(dtype, A, W2, S, C, Other, Bias, M, N, K, postop, out_f32, st);
 }
 

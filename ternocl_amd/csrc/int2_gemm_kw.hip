@@ -128,7 +128,7 @@ KwPlan kw_plan(int M, int N, int K, bool split) {
         if (t.bm > 32 && t.bm >= 2 * M) continue;  // half the tile's rows idle: a lower one does it
         const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
         for (int ks = 1; ks <= 8; ++ks) {
-            if (ks > 1 && (!split || K / ks < 512 || tiles * 4 > (long)kWsHeader)) break;
+            if (ks > 1 && (!split || K / ks < 512 || tiles * ks > 1024 || tiles * 4 > (long)kWsHeader)) break;
             const double rounds = (double)((tiles * ks + 255) / 256);
             double us = t.base * (0.5 + 0.5 * rounds) + t.slope * rounds * K / (1024.0 * ks);
             if (ks > 1) us += 1.2 + 8e-6 * ks * M * N / 4.0;
@@ -170,35 +170,42 @@ void int2_gemm_kw_model(int M, int N, int K, bool bf, double &kw_us, double &oth
     wk = p.tile <= 1 ? 8 : 4;
 }
 
-// Whether the automatic engine of a call of M > 8 rows is this one: always up
-// to 16 rows (the MFMA GEMV is 2-3x its time there), above where its model is
-// ahead of the 128-row tile engine's.  split: whether K slices may use a
-// workspace.
-static bool kw_wins(int M, int N, int K, bool split, bool bf) {
-    return M <= 16 || (M <= 2048 && kw_plan(M, N, K, split).us < kKwMargin * kw_other_us(M, N, K, split, bf));
-}
-// (the vector loads and stores need 16-byte aligned operands)
-bool int2_gemm_kw_auto(int M, int N, int K, bool split, bool bf, const void *A, const void *B, const void *S, const void *C,
-                       const void *Other, const void *Bias) {
-    return M > 8 && aligned16(A) && aligned16(B) && aligned16(S) && aligned16(C) && aligned16(Other) && aligned16(Bias) &&
-           kw_wins(M, N, K, split, bf);
+// Whether plan p is the automatic engine of a call of M > 8 rows: always up to 16
+// rows (the MFMA GEMV is 2-3x its time there), above where its model is ahead of
+// the 128-row tile engine's.  split: whether K slices may use a workspace.
+static bool kw_wins(const KwPlan &p, int M, int N, int K, bool split, bool bf) {
+    return M <= 16 || (M <= 2048 && p.us < kKwMargin * kw_other_us(M, N, K, split, bf));
 }
 
 // Workspace of the automatic plan's K split (0: none; none up to 16 rows).
 size_t int2_gemm_kw_ws_need(int M, int N, int K) {
     if (M <= 16 || M > 2048) return 0;
     const KwPlan p = kw_plan(M, N, K, true);
-    return p.ks > 1 && (kw_wins(M, N, K, true, false) || kw_wins(M, N, K, true, true)) ? kWsHeader + (size_t)p.ks * M * N * 4 : 0;
+    if (p.ks == 1 || !(kw_wins(p, M, N, K, true, false) || kw_wins(p, M, N, K, true, true))) return 0;
+    return kWsHeader + (size_t)p.ks * M * N * 4;
 }
 
-// split: K slices may use ws (int2_gemm_kw_ws_need bytes, 16-byte aligned).
-ternocl_status int2_gemm_kw_run(int dtype, const void *A, const uint32_t *B, const void *S, void *C, const void *Other,
-                                const void *Bias, int M, int N, int K, int postop, int out_f32, hipStream_t st,
-                                bool split, void *ws) {
-    const KwPlan p = kw_plan(M, N, K, split && M > 16);
+// Runs the call here if this is its automatic engine (force: whichever the
+// models prefer) and returns whether it did; the status in s.  A K split needs
+// its slice sums in ws; with less the unsplit plan is weighed.  The vector
+// loads and stores need 16-byte aligned operands.
+bool int2_gemm_kw_run(int dtype, const void *A, const uint32_t *B, const void *S, void *C, const void *Other,
+                      const void *Bias, int M, int N, int K, int postop, int out_f32, hipStream_t st, void *ws,
+                      size_t ws_bytes, bool force, ternocl_status &s) {
+    const bool bf = dtype == TERNOCL_BF16;
+    if (M <= 8 || M > 2048 || !aligned16(A) || !aligned16(B) || !aligned16(S) || !aligned16(C) || !aligned16(Other) ||
+        !aligned16(Bias))
+        return false;
+    const bool ws_ok = ws && ws_bytes > kWsHeader && aligned16(ws) && M > 16;
+    KwPlan p = kw_plan(M, N, K, ws_ok);
+    bool split = ws_ok;
+    if (p.ks > 1 && ws_bytes < kWsHeader + (size_t)p.ks * M * N * 4) {
+        p = kw_plan(M, N, K, false);
+        split = false;
+    }
+    if (!force && !kw_wins(p, M, N, K, split, bf)) return false;
     uint32_t *cnt = p.ks > 1 ? (uint32_t *)ws : nullptr;
     float *part = p.ks > 1 ? (float *)((uint8_t *)ws + kWsHeader) : nullptr;
-    const bool bf = dtype == TERNOCL_BF16;
     auto go = [&](auto cfg) {
         typedef decltype(cfg) Cfg;
         return bf ? kw_launch<Cfg, true>(A, B, S, C, Other, Bias, M, N, K, postop, out_f32, p.ks, part, cnt, st)
@@ -213,7 +220,8 @@ ternocl_status int2_gemm_kw_run(int dtype, const void *A, const uint32_t *B, con
     case 4: e = go(KwCfg<2, 4, 1, 4, 2>{}); break;
     default: e = go(KwCfg<2, 4, 2, 4, 2>{}); break;
     }
-    return launch_status(e);
+    s = launch_status(e);
+    return true;
 }
 
 }  // namespace tcl

@@ -46,12 +46,9 @@ namespace tcl {
 int gemm_splits(int M, int N, int K);
 bool gemm_half_tile(int M, int N);
 // (int2_int8_kw.hip)
-bool int2_int8_kw_auto(int M, int N, int K, bool split, const void *A, const void *B, const void *SB, const void *C,
-                       const void *Other, const void *Bias);
-size_t int2_int8_kw_ws_need(int M, int N, int K);
-hipError_t int2_int8_kw_run(int dtype, const void *A, const int8_t *Aq, const void *SA, const uint32_t *B, const void *SB,
-                            void *C, const void *Other, const void *Bias, int M, int N, int K, int postop, int out_f32,
-                            hipStream_t st, bool split, void *ws);
+bool int2_int8_kw_run(int dtype, const void *A, const int8_t *Aq, const void *SA, const uint32_t *B, const void *SB,
+                      void *C, const void *Other, const void *Bias, int M, int N, int K, int postop, int out_f32,
+                      hipStream_t st, void *ws, size_t ws_bytes, hipError_t &e);
 hipError_t splitk_reduce_launch(int dtype, const float *part, int splits, void *C, const void *Other,
                                 const void *Bias, int M, int N, int postop, int out_f32, hipStream_t st);
 namespace {
@@ -846,10 +843,9 @@ ternocl_status int2_int8_gemm_run(int dtype, const void *A, const int8_t *Aq, co
         return TERNOCL_ERR_UNSUPPORTED_SHAPE;
     }
     // few to hundreds of rows: K split over the waves where that model is ahead
-    const size_t kw_need = int2_int8_kw_ws_need(M, N, K);
-    const bool kw_split = kw_need && ws && ((uintptr_t)ws & 15) == 0 && ws_bytes >= kw_need;
-    if (int2_int8_kw_auto(M, N, K, kw_split, Aq ? (const void *)Aq : A, B, SB, C, Other, Bias))
-        return launch_status(int2_int8_kw_run(dtype, A, Aq, SA, B, SB, C, Other, Bias, M, N, K, postop, out_f32, st, kw_split, ws));
+    hipError_t kw_e;
+    if (int2_int8_kw_run(dtype, A, Aq, SA, B, SB, C, Other, Bias, M, N, K, postop, out_f32, st, ws, ws_bytes, kw_e))
+        return launch_status(kw_e);
     // 128 x 256 tiles of eight 128 x 32 waves where 128 x 128 tiles would
     // number more than 256 and 128 x 256 tiles fit one per CU (the fp16
     // prefill GEMM's rule): they decode each weight word for 128 rows, the

@@ -265,7 +265,7 @@ I8Plan i8kw_plan(int M, int N, int K, bool split) {
         if (t.bm > 32 && t.bm >= 2 * M) continue;  // half the tile's rows idle
         const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
         for (int ks = 1; ks <= 8; ++ks) {
-            if (ks > 1 && (!split || K / ks < 512 || tiles * 4 > (long)kWsHeader)) break;
+            if (ks > 1 && (!split || K / ks < 512 || tiles * ks > 1024 || tiles * 4 > (long)kWsHeader)) break;
             double us = i8kw_us(i, (double)tiles * ks, K / (1024.0 * ks));
             if (ks > 1) us += 1.2 + 8e-6 * ks * M * N / 4.0;
             if (us < best.us - 1e-9) best = {i, ks, us};
@@ -294,30 +294,35 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
 
-// Whether a call of M > 4 rows takes this engine (split: whether K slices may use
-// a workspace); the same answer in both quantization modes, whose bits agree.
-// The vector loads and stores need 16-byte aligned operands.
-bool int2_int8_kw_auto(int M, int N, int K, bool split, const void *A, const void *B, const void *SB, const void *C,
-                       const void *Other, const void *Bias) {
-    if (M < 1 || M > 2048 || !aligned16(A) || !aligned16(B) || !aligned16(SB) || !aligned16(C) || !aligned16(Other) ||
-        !aligned16(Bias))
-        return false;
-    return i8kw_plan(M, N, K, split).us < kI8Margin * i8_other_us(M, N, K, split);
+static bool i8kw_wins(const I8Plan &p, int M, int N, int K, bool split) {
+    return p.us < kI8Margin * i8_other_us(M, N, K, split);
 }
 
 // Workspace of the automatic plan's K split (0: none).
 size_t int2_int8_kw_ws_need(int M, int N, int K) {
     if (M <= 4 || M > 2048) return 0;
     const I8Plan p = i8kw_plan(M, N, K, true);
-    return p.ks > 1 && p.us < kI8Margin * i8_other_us(M, N, K, true) ? kWsHeader + (size_t)p.ks * M * N * 4 : 0;
+    return p.ks > 1 && i8kw_wins(p, M, N, K, true) ? kWsHeader + (size_t)p.ks * M * N * 4 : 0;
 }
 
-// Aq non-null: upfront mode, else A's DT rows.  split: K slices may use ws
-// (int2_int8_kw_ws_need bytes, 16-byte aligned).
-hipError_t int2_int8_kw_run(int dtype, const void *A, const int8_t *Aq, const void *SA, const uint32_t *B, const void *SB,
-                            void *C, const void *Other, const void *Bias, int M, int N, int K, int postop, int out_f32,
-                            hipStream_t st, bool split, void *ws) {
-    const I8Plan p = i8kw_plan(M, N, K, split);
+// Runs the call here if the models prefer this engine and returns whether it
+// did; the error in e.  Aq non-null: upfront mode, else A's DT rows; the choice
+// is the same in both, whose bits agree.  A K split needs its slice sums in ws;
+// with less the unsplit plan is weighed.  The vector loads and stores need
+// 16-byte aligned operands.
+bool int2_int8_kw_run(int dtype, const void *A, const int8_t *Aq, const void *SA, const uint32_t *B, const void *SB,
+                      void *C, const void *Other, const void *Bias, int M, int N, int K, int postop, int out_f32,
+                      hipStream_t st, void *ws, size_t ws_bytes, hipError_t &e) {
+    if (M > 2048 || !aligned16(Aq ? (const void *)Aq : A) || !aligned16(B) || !aligned16(SB) || !aligned16(C) ||
+        !aligned16(Other) || !aligned16(Bias))
+        return false;
+    bool split = ws && ws_bytes > kWsHeader && aligned16(ws);
+    I8Plan p = i8kw_plan(M, N, K, split);
+    if (p.ks > 1 && ws_bytes < kWsHeader + (size_t)p.ks * M * N * 4) {
+        p = i8kw_plan(M, N, K, false);
+        split = false;
+    }
+    if (!i8kw_wins(p, M, N, K, split)) return false;
     uint32_t *cnt = p.ks > 1 ? (uint32_t *)ws : nullptr;
     float *part = p.ks > 1 ? (float *)((uint8_t *)ws + kWsHeader) : nullptr;
     auto go = [&](auto cfg) {
@@ -331,11 +336,12 @@ hipError_t int2_int8_kw_run(int dtype, const void *A, const int8_t *Aq, const vo
         return Aq ? one(std::false_type{}, std::false_type{}) : one(std::false_type{}, std::true_type{});
     };
     switch (p.tile) {
-    case 0: return go(KwCfg<1, 1, 1, 8>{});
-    case 1: return go(KwCfg<1, 2, 1, 8>{});
-    case 2: return go(KwCfg<1, 2, 1, 4>{});
-    default: return go(KwCfg<1, 2, 2, 4>{});
+    case 0: e = go(KwCfg<1, 1, 1, 8>{}); break;
+    case 1: e = go(KwCfg<1, 2, 1, 8>{}); break;
+    case 2: e = go(KwCfg<1, 2, 1, 4>{}); break;
+    default: e = go(KwCfg<1, 2, 2, 4>{}); break;
     }
+    return true;
 }
 
 }  // namespace tcl
