@@ -106,6 +106,24 @@ template <int CB, int PF> struct KwInt2 {
     }
 };
 
+// Two matrices of the same shape side by side (the MoE layer's up and gate): the
+// lane's first CB / 2 column blocks are a's columns, the others b's same columns.
+template <int CB, int PF> struct KwDual {
+    KwInt2<CB / 2, PF> a, b;
+    __device__ __forceinline__ void start(int u0) {
+        a.start(u0);
+        b.start(u0);
+    }
+    __device__ __forceinline__ void next(int u, int s, bool more) {
+        a.next(u, s, more);
+        b.next(u, s, more);
+    }
+    __device__ __forceinline__ void get(int s, uint32_t w[CB][2], uint32_t lo[CB], uint32_t hi[CB]) {
+        a.get(s, w, lo, hi);
+        b.get(s, w + CB / 2, lo + CB / 2, hi + CB / 2);
+    }
+};
+
 // The K walk of one wave: units [u0, u1) (64 rows of K each) of its 32 MB rows
 // into acc.  abuf: the wave's LDS (two units); A + va[i] (elements) + 64 u: the
 // 16-byte chunk lane % 8 of its row i * 8 + lane / 8.
@@ -228,28 +246,42 @@ __device__ __forceinline__ void kw_store(void *C, const uint16_t *Other, const v
 // m0) and columns [n0, n0 + 32 CB) (below N).  ksn > 1: slice sl's sums go to part
 // [ksn][M][N] (agent-scope stores), and the last of the tile's ksn workgroups
 // (its counter cnt, split_arrive) adds the slices in order -- the handoff of the
-// decode GEMV's K split (int2_gemv_f4.hip).
-template <class Cfg, bool BF16>
+// decode GEMV's K split (int2_gemv_f4.hip).  DUAL (KwDual's sums, ksn == 1): C =
+// DT(silu(gate) * DT(up)) on CB / 2 columns a lane, the bits of the up product
+// stored in DT and read by the gate product's epilogue.
+template <class Cfg, bool BF16, bool DUAL = false>
 __device__ __forceinline__ void kw_finish(f32x16_t acc[Cfg::MB][Cfg::CB], uint8_t *lds, void *C, const uint16_t *Other,
                                           const void *Bias, int M, int N, int m0, int mrows, int n0, int postop, int out_f32,
                                           int ksn, int sl, float *part, uint32_t *cnt) {
-    constexpr int MB = Cfg::MB, CB = Cfg::CB, WK = Cfg::WK;
+    constexpr int MB = Cfg::MB, CB = Cfg::CB, WK = Cfg::WK, CS = DUAL ? CB / 2 : CB;
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, q = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kw = wave / Cfg::WM, wm = wave % Cfg::WM;
     auto rows_of = [&](int it, int &r, int &n) __attribute__((always_inline)) {
         // item `it` of a round: row block it / 256, register quad (it / 64) % 4, this lane
         r = 32 * (it >> 8) + 8 * ((it >> 6) & 3) + 4 * q;
-        n = n0 + CB * c;
+        n = n0 + CS * c;
     };
     auto finish = [&](int r, int n, const float (*v)[4]) __attribute__((always_inline)) {
+        if constexpr (DUAL) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (r + i < mrows && n < N) {
+                    float x[CS];
+#pragma unroll
+                    for (int cb = 0; cb < CS; ++cb)
+                        x[cb] = epi_apply_c<1>(v[CS + cb][i], dt2f<BF16>(f2dt<BF16>(v[cb][i])), 0.0f);
+                    kw_store<CS, BF16, 0, false>(C, nullptr, nullptr, N, m0 + r + i, n, x);
+                }
+            return;
+        }
         epi_dispatch(postop, out_f32, [&](auto P_, auto F_) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 if (r + i < mrows && n < N) {
-                    float x[CB];
+                    float x[CS];
 #pragma unroll
-                    for (int cb = 0; cb < CB; ++cb) x[cb] = v[cb][i];
-                    kw_store<CB, BF16, decltype(P_)::value, decltype(F_)::value>(C, Other, Bias, N, m0 + r + i, n, x);
+                    for (int cb = 0; cb < CS; ++cb) x[cb] = v[cb][i];
+                    kw_store<CS, BF16, decltype(P_)::value, decltype(F_)::value>(C, Other, Bias, N, m0 + r + i, n, x);
                 }
         });
     };

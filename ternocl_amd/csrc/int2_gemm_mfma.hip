@@ -30,6 +30,10 @@
 #include "common.hpp"
 
 namespace tcl {
+// (moe_kw.hip: experts of few rows)
+bool moe_gemm_kw_run(int dtype, const int *meta, const void *A, const int *perm, int topk, const uint32_t *B, const void *S,
+                     const uint32_t *B2, const void *S2, void *C, const void *Other, int E, int G, int N, int K, int postop,
+                     int out_f32, hipStream_t st, ternocl_status &s);
 // Whether a prefill GEMM below the 128 x 512 tile's 192-tile mark runs 128 x
 // 256 tiles: where 128 x 128 tiles would number more than 256 (some CUs would
 // hold two) and 128 x 256 tiles fit one per CU.  Used by gemm_plan (the
@@ -898,6 +902,10 @@ ternocl_status moe_gemm_run(int dtype, const int *meta, const void *A_all, const
     typedef TileCfg<4, 2, 2, 4> W128;
     typedef TileCfg<4, 8, 2, 4> P512;  // pair tiles: 2 x 4 waves of 64 rows, the same columns
     typedef TileCfg<4, 4, 2, 4> P256;
+    ternocl_status s;
+    if (moe_gemm_kw_run(dtype, meta, A_all, perm, topk, B_all, S_all, nullptr, nullptr, C_all, Other_all, E, G, N, K, postop,
+                        out_f32, st, s))
+        return s;
     const int bn = moe_bn(N, 512);
     if (dtype == TERNOCL_BF16) {
         if (desc) {  // the layer's tile list: two experts' tails may share a tile
@@ -930,6 +938,8 @@ ternocl_status moe_gate_up_run(int dtype, const int *meta, const void *A_all, co
     typedef TileCfg<8, 2, 1, 8> W256;
     typedef TileCfg<4, 2, 2, 4> W128;
     typedef TileCfg<4, 4, 2, 4> P256;  // pair tiles: 2 x 4 waves of 64 rows, the same columns
+    ternocl_status s;
+    if (moe_gemm_kw_run(dtype, meta, A_all, perm, topk, Bu, Su, Bg, Sg, Hs, nullptr, E, G, N, K, 1, 0, st, s)) return s;
     const bool wide = moe_bn(N, 256) == 256;
     if (desc) {  // the layer's tile list: two experts' tails may share a tile
         if (dtype == TERNOCL_BF16) {
