@@ -79,10 +79,20 @@ def _ptr(x) -> int | None:
     return x.data_ptr()
 
 
+def _current_stream() -> int:
+    """The handle of torch's current stream on the current device.  torch's raw accessors (0.1 us each)
+    where it has them: torch.cuda.current_stream() builds a Stream object, 3.0 us of the 8.3 us a decode
+    call took on the host (5.3 us with them, of which the launch is 3.9)."""
+    import torch
+    c = torch._C
+    if hasattr(c, "_cuda_getCurrentRawStream") and torch.cuda.is_initialized():
+        return c._cuda_getCurrentRawStream(c._cuda_getDevice())
+    return torch.cuda.current_stream().cuda_stream
+
+
 def _stream(stream) -> int | None:
     if stream is None:
-        import torch
-        return torch.cuda.current_stream().cuda_stream
+        return _current_stream()
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream

@@ -170,3 +170,20 @@ def test_moe_ops_match_direct_calls(dev, Tk, decode):
         T.int2_moe_prefill(X, ids, RW, Tk, E, topk, H, I, Bg, Sg, Bu, Su, Bd, Sd, O, ws)
     torch.cuda.synchronize()
     assert np.array_equal(host_u16(got), host_u16(O))
+
+
+@pytest.mark.gpu
+def test_calls_follow_the_current_stream(dev):
+    """A call without a stream argument launches on torch's current stream, the default one and a side
+    stream: work queued before it there is seen by it."""
+    import torch
+    import ternocl_amd as T
+    assert T._stream(None) == torch.cuda.current_stream().cuda_stream
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert T._stream(None) == side.cuda_stream
+        ws = torch.ones(1 << 20, dtype=torch.uint8, device="cuda")
+        T.workspace_zero(ws)
+    side.synchronize()
+    assert not ws.any().item()
+    assert T._stream(None) == torch.cuda.current_stream().cuda_stream
