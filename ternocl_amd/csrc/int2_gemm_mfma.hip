@@ -608,15 +608,44 @@ __device__ __forceinline__ void gemm_tile(const ARows &ar, uint32_t a_bytes, int
 // [s K / splits, (s + 1) K / splits) and writes its fp32 partial tile into
 // part + s M N (no epilogue); k_splitk_reduce adds the slices in order.  The
 // slices of a tile are adjacent in the XCD order, so they share its A rows.
-template <class Cfg, bool BF16>
+// TCfg (not void): the launch's first `full` workgroups take whole tiles, and each tile
+// after those is cut into Cfg::BN / TCfg::BN column tiles of TCfg's, so the last
+// round keeps every CU busy (gemm_tail).  The sums of an output do not depend on
+// the tile.
+template <class Cfg, bool BF16, class TCfg = void>
 __global__ void __launch_bounds__(Cfg::THREADS)
 k_int2_gemm(const uint16_t *__restrict__ A, const uint32_t *__restrict__ B,
             const uint16_t *__restrict__ S, void *__restrict__ C, const uint16_t *__restrict__ Other,
             const void *__restrict__ Bias, int M, int N, int K, int postop, int out_f32, int splits = 1,
-            float *__restrict__ part = nullptr) {
+            float *__restrict__ part = nullptr, int full = 0) {
     __shared__ __attribute__((aligned(16))) uint16_t lds[Cfg::lds_elems];
     const int mt = (M + Cfg::BM - 1) / Cfg::BM, nt = (N + Cfg::BN - 1) / Cfg::BN;
     int tm, tns;
+    if constexpr (!std::is_void_v<TCfg>) {
+        static_assert(TCfg::THREADS == Cfg::THREADS && TCfg::BM == Cfg::BM && Cfg::BN % TCfg::BN == 0 &&
+                      TCfg::lds_elems <= Cfg::lds_elems, "a tail tile fits the launch");
+        constexpr int CUT = Cfg::BN / TCfg::BN;
+        int t, sub = 0;
+        if ((int)blockIdx.x < full) {
+            t = (blockIdx.x & 7) * (full / 8) + (blockIdx.x >> 3);  // (full: a multiple of 256)
+        } else {
+            int row, u;
+            if (!xcd_tile_ashare(blockIdx.x - full, 1, (mt * nt - full) * CUT, row, u)) return;  // padding
+            t = full + u / CUT;
+            sub = u % CUT;
+        }
+        tm = __builtin_amdgcn_readfirstlane(t / nt);
+        const int n0 = __builtin_amdgcn_readfirstlane((t - tm * nt) * Cfg::BN + sub * TCfg::BN);
+        if (n0 >= N) return;  // whole workgroup
+        const ARows ar{A + (size_t)tm * Cfg::BM * K, nullptr, 1};
+        const int mrows = min(Cfg::BM, M - tm * Cfg::BM);
+        const uint32_t a_bytes = (uint32_t)((size_t)mrows * K * 2);
+        if ((int)blockIdx.x < full)
+            gemm_tile<Cfg, BF16>(ar, a_bytes, mrows, B, S, C, Other, Bias, tm * Cfg::BM, N, K, K, n0, postop, out_f32, lds);
+        else
+            gemm_tile<TCfg, BF16>(ar, a_bytes, mrows, B, S, C, Other, Bias, tm * Cfg::BM, N, K, K, n0, postop, out_f32, lds);
+        return;
+    }
     if (!xcd_tile_ashare(blockIdx.x, mt, nt * splits, tm, tns)) return;  // whole workgroup: padding
     // (uniform: kept in scalar registers, so the buffer descriptors built
     // from them stay scalar -- a divided value otherwise reads as per-lane)
@@ -823,11 +852,37 @@ void gemm_launch(const void *A, const uint32_t *B, const void *S, void *C, const
                        postop, out_f32);
 }
 
+// Wide tiles past the last whole round of 256 (one workgroup a CU).  A last round
+// of at most 64 of them runs as 128 x 128 tiles (four times as many), of at most
+// 128 as 128 x 256 tiles: one round of those takes 0.45 / 0.65 of the wide one.
+// bf16 / fp16, same box, us: M = 2048 K = 5120 N = 34816 (1088 tiles) 638.8 / 614.5 ->
+// 597.5 / 599.2, M = 1024 (544) 357.7 / 355.6 -> 317.9 / 316.0, M = 1024 K = 4096 N =
+// 18432 (288) 186.5 / 184.5 -> 146.2 / 145.5, M = 700 N = 25600 (300) 186.7 / 184.6 ->
+// 144.6 / 150.7; 128 x 256: M = 1024 K = 5376 N = 21504 (336) 242.9 / 238.9 -> 222.4 /
+// 221.4.  Past 128 a second round of halves would cost more than the wide one.
+int gemm_tail(int M, int N) { return (int)(((long)((M + 127) / 128) * ((N + 511) / 512)) % 256); }
+
+template <class TCfg, bool BF16>
+void gemm_launch_tail(const void *A, const uint32_t *B, const void *S, void *C, const void *Other, const void *Bias,
+                      int M, int N, int K, int postop, int out_f32, int tail, hipStream_t st) {
+    typedef TileCfg<8, 4, 1, 8> Cfg;
+    const int full = ((M + Cfg::BM - 1) / Cfg::BM) * ((N + Cfg::BN - 1) / Cfg::BN) - tail;
+    hipLaunchKernelGGL((k_int2_gemm<Cfg, BF16, TCfg>), dim3(full + xcd_ashare_grid(1, tail * (Cfg::BN / TCfg::BN))),
+                       dim3(Cfg::THREADS), 0, st, (const uint16_t *)A, B, (const uint16_t *)S, C, (const uint16_t *)Other,
+                       Bias, M, N, K, postop, out_f32, 1, nullptr, full);
+}
+
 template <bool BF16>
 void gemm_dispatch(const GemmPlan &p, const void *A, const uint32_t *B, const void *S, void *C,
                    const void *Other, const void *Bias, int M, int N, int K, int postop, int out_f32,
                    hipStream_t st) {
-    if (p.wvn == 8 && p.ncb == 4) gemm_launch<TileCfg<8, 4, 1, 8>, BF16>(A, B, S, C, Other, Bias, M, N, K, postop, out_f32, st);
+    const int tail = gemm_tail(M, N);
+    const bool wide = p.wvn == 8 && p.ncb == 4 && (long)((M + 127) / 128) * ((N + 511) / 512) >= 256;
+    if (wide && tail > 0 && tail <= 64)
+        gemm_launch_tail<TileCfg<4, 2, 2, 4>, BF16>(A, B, S, C, Other, Bias, M, N, K, postop, out_f32, tail, st);
+    else if (wide && tail > 64 && tail <= 128)
+        gemm_launch_tail<TileCfg<8, 2, 1, 8>, BF16>(A, B, S, C, Other, Bias, M, N, K, postop, out_f32, tail, st);
+    else if (p.wvn == 8 && p.ncb == 4) gemm_launch<TileCfg<8, 4, 1, 8>, BF16>(A, B, S, C, Other, Bias, M, N, K, postop, out_f32, st);
     else if (p.wvn == 8) gemm_launch<TileCfg<8, 2, 1, 8>, BF16>(A, B, S, C, Other, Bias, M, N, K, postop, out_f32, st);
     else gemm_launch<TileCfg<4, 2, 2, 4>, BF16>(A, B, S, C, Other, Bias, M, N, K, postop, out_f32, st);
 }
