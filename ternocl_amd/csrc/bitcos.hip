@@ -126,15 +126,7 @@ __device__ __forceinline__ void bc_fwht_block(const uint16_t *__restrict__ x, co
                 v[j] = a + c;
                 v[j + h] = a - c;
             }
-    for (int h = 8; h < n; h <<= 1) {  // partner lane ^ h / 8 holds elements i ^ h
-        const int m = h >> 3;
-        const bool up = (lane & m) != 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float p = __shfl_xor(v[j], m);
-            v[j] = up ? p - v[j] : v[j] + p;  // (a + c, a - c) with a the lower element
-        }
-    }
+    fwht_wave(v, n, lane);
     if (!live) return;
     uint32_t o[4];
 #pragma unroll

@@ -110,6 +110,46 @@ __device__ __forceinline__ uint32_t split_arrive(uint32_t *c, int ksn, int lane)
     return __builtin_amdgcn_readfirstlane(prev);
 }
 
+// The value of lane ^ M (M a power of two below 64): DPP moves for 1, 2, 4 and 8, the
+// row and half swaps for 16 and 32, all VALU; __shfl_xor's ds_bpermute goes through
+// LDS.  The aligned lanes that it moves among must be active.
+template <int M> __device__ __forceinline__ float lane_xor(float v, int lane) {
+    const int x = __float_as_int(v);
+    if constexpr (M == 1) return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0xB1, 0xf, 0xf, true));  // quad [1, 0, 3, 2]
+    else if constexpr (M == 2) return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0x4E, 0xf, 0xf, true));  // [2, 3, 0, 1]
+    else if constexpr (M == 4) {  // half-row mirror (lane ^ 7), then the quad's (lane ^ 3)
+        const int y = __builtin_amdgcn_mov_dpp(x, 0x141, 0xf, 0xf, true);
+        return __int_as_float(__builtin_amdgcn_mov_dpp(y, 0x1B, 0xf, 0xf, true));
+    } else if constexpr (M == 8) return __int_as_float(__builtin_amdgcn_mov_dpp(x, 0x128, 0xf, 0xf, true));  // row rotate 8
+    else if constexpr (M == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);  // even rows' values, odd rows' values
+        return __uint_as_float((lane & 16) ? r[0] : r[1]);
+    } else {
+        static_assert(M == 32, "a lane of the wave");
+        const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);  // the lower, the upper half's values
+        return __uint_as_float((lane & 32) ? r[0] : r[1]);
+    }
+}
+// The transform's stage between lane and lane ^ M on 8 elements a lane: (a + c, a -
+// c) with a the lower lane's.
+template <int M> __device__ __forceinline__ void fwht_lanes(float v[8], int lane) {
+    const bool up = (lane & M) != 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float p = lane_xor<M>(v[j], lane);
+        v[j] = up ? p - v[j] : v[j] + p;
+    }
+}
+// Its stages of stride 8 .. min(n, 512) / 2 (n a uniform power of two), in order.
+__device__ __forceinline__ void fwht_wave(float v[8], int n, int lane) {
+    if (n > 8) fwht_lanes<1>(v, lane);
+    if (n > 16) fwht_lanes<2>(v, lane);
+    if (n > 32) fwht_lanes<4>(v, lane);
+    if (n > 64) fwht_lanes<8>(v, lane);
+    if (n > 128) fwht_lanes<16>(v, lane);
+    if (n > 256) fwht_lanes<32>(v, lane);
+}
+
 // c + w.lo * a.lo + w.hi * a.hi on packed DT pairs (v_dot2_f32_{f16,bf16})
 template <bool BF16>
 __device__ __forceinline__ float dot2(uint32_t w, uint32_t a, float c) {

@@ -14,13 +14,18 @@
 //  * k_fwht_r (16-byte aligned x and y, K % 8 == 0, a tail block of 0 or >= 8
 //    elements): thread t holds elements 8t .. 8t + 7 of its block in
 //    registers; strides 1, 2, 4 run in registers, 8 .. 256 between the lanes
-//    of a wave (lane xor stride / 8), 512 and up between the waves of the
-//    workgroup through LDS.  One 16-byte load and store per thread; a 512-block
-//    needs no barrier at all.
+//    of a wave (lane xor stride / 8: DPP and lane swaps, no LDS); blocks of 1024
+//    and up pass LDS once, after which a thread holds the elements 512 apart of
+//    its positions and runs the last strides in registers.  A 512-block needs no
+//    barrier at all.  fp16, with two barriers and an LDS round trip of 32-byte
+//    lane strides a stride from 512 up and bpermutes between lanes -> so: HB
+//    4096, 1 x 8192 6.1 -> 3.3 us, 1024 x 8192 33.2 -> 12.1 (2.8 TB/s), 8192 x
+//    8192 230 -> 78 (3.5 TB/s); HB 1024, 300 x 8192 7.8 -> 5.7; HB 512, 300 x
+//    5376 4.57 -> 4.40, 8192 x 5376 51 -> 45 (3.9 TB/s).
 //  * k_fwht (any other case): one workgroup of 256 threads per block, the
 //    block in LDS as fp32, one barrier per stage.
 // Both are latency-bound at the sizes of a decode step (one row of a few
-// thousand elements).
+// thousand elements); k_fwht_r nears the copy rate (5.2 TB/s) at thousands of rows.
 #include "common.hpp"
 
 namespace tcl {
@@ -96,36 +101,47 @@ k_fwht_r(const uint16_t *__restrict__ x, const int8_t *__restrict__ signs, uint1
                 v[j] = a + c;
                 v[j + h] = a - c;
             }
-    for (int h = 8; h < n && h < 512; h <<= 1) {  // partner lane ^ h / 8 holds elements i ^ h
-        const int m = h >> 3;
-        const bool up = (lane & m) != 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const float p = __shfl_xor(v[j], m);
-            v[j] = up ? p - v[j] : v[j] + p;  // (a + c, a - c) with a the lower element
-        }
-    }
-    for (int h = 512; h < n; h <<= 1) {  // partner thread t ^ h / 8, through LDS
+    fwht_wave(v, n, lane);
+    const float sc = n == HB ? scale_full : scale_tail;
+    uint16_t *yb = y + (size_t)row * K + k0;
+    if (n >= 1024) {  // (uniform) strides 512 and up: thread t takes elements p + 512 w of its positions p
         if (live)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) xw[e0 + j] = v[j];
+            for (int j = 0; j < 8; j += 4) *(float4 *)(xw + e0 + j) = make_float4(v[j], v[j + 1], v[j + 2], v[j + 3]);
         __syncthreads();
-        const bool up = (e0 & h) != 0;
-        if (live)
+        if (!live) return;
+        auto across = [&](auto W_) __attribute__((always_inline)) {
+            constexpr int W = decltype(W_)::value;  // 512-element parts of the block
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float p = xw[(e0 ^ h) + j];
-                v[j] = up ? p - v[j] : v[j] + p;
+            for (int k = 0; k < 8 / W; ++k) {
+                const int p = t + 64 * W * k;
+                float u[W];
+#pragma unroll
+                for (int w = 0; w < W; ++w) u[w] = xw[512 * w + p];
+#pragma unroll
+                for (int h = 1; h < W; h <<= 1)
+#pragma unroll
+                    for (int w = 0; w < W; ++w)
+                        if ((w & h) == 0) {
+                            const float a = u[w], c = u[w + h];
+                            u[w] = a + c;
+                            u[w + h] = a - c;
+                        }
+#pragma unroll
+                for (int w = 0; w < W; ++w) yb[512 * w + p] = (uint16_t)f2dt<BF16>(u[w] * sc);
             }
-        __syncthreads();
+        };
+        if (n == 1024) across(std::integral_constant<int, 2>{});
+        else if (n == 2048) across(std::integral_constant<int, 4>{});
+        else across(std::integral_constant<int, 8>{});
+        return;
     }
     if (!live) return;
-    const float sc = n == HB ? scale_full : scale_tail;
     uint32_t o[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
         o[i] = (uint32_t)f2dt<BF16>(v[2 * i] * sc) | ((uint32_t)f2dt<BF16>(v[2 * i + 1] * sc) << 16);
-    *(uint4 *)(y + (size_t)row * K + k0 + e0) = make_uint4(o[0], o[1], o[2], o[3]);
+    *(uint4 *)(yb + e0) = make_uint4(o[0], o[1], o[2], o[3]);
 }
 
 }  // namespace
