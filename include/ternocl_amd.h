@@ -135,6 +135,20 @@ ternocl_status ternocl_int2_fp16_upcvt_gemm_ex(int dtype, const void *A, const u
                                                int postop, int out_f32, void *ws,
                                                size_t ws_bytes, const ternocl_gemv_tile *tile,
                                                void *stream);
+/* Host-side test hook, no device work: whether an automatic call on 16-byte
+ * aligned operands runs a GEMM that splits K over the waves of a workgroup (1;
+ * 0: another engine), and its tile.  entry: 0 ternocl_int2_fp16_upcvt_gemm with
+ * ws_bytes of workspace (0: none), 1 ternocl_int2_int8_gemm_ws, 2
+ * ternocl_bitcos_fp16_upcvt_gemm_mt, 3 one product of M assignments over E
+ * experts in ternocl_int2_moe_gemm / _prefill. */
+typedef struct {
+    int rows, cols; /* output tile of a workgroup */
+    int k_waves;    /* waves over K */
+    int k_slices;   /* workgroups over K (> 1: sums in the workspace) */
+    int repacked;   /* entry 2: with a workspace the weights are re-packed first */
+} ternocl_kw_tile;
+int ternocl_kw_tile_of(int entry, int dtype, int M, int N, int K, int E, size_t ws_bytes, ternocl_kw_tile *tile);
+
 /* Zero-fill device memory with a fill kernel (no hipMemset: graph-capturable). */
 ternocl_status ternocl_workspace_zero(void *ws, size_t ws_bytes, void *stream);
 

@@ -21,7 +21,7 @@ from . import _abi
 
 __all__ = [
     "TernoclError", "lib", "library_path", "FP16", "BF16", "WS_HEADER_BYTES",
-    "int2_gemm_ws_bytes", "workspace_zero", "int2_fp16_upcvt_gemm", "int2_dequant",
+    "int2_gemm_ws_bytes", "workspace_zero", "kw_tile_of", "int2_fp16_upcvt_gemm", "int2_dequant",
     "int2_gemv_decode", "int2_gemv_stream_probe", "stream_read_probe", "gemv_tile", "GemvTile", "VALU", "MFMA", "GEMM",
     "int2_pack", "int2_unpack", "bitcos_pack", "bitcos_unpack", "bitcos_slice_ranks_host",
     "ldsa", "quant_a", "int2_int8_gemm", "int2_int8_gemm_ws_bytes", "int2_s8_decode",
@@ -116,6 +116,15 @@ def _nbytes(t) -> int:
 def int2_gemm_ws_bytes(M: int, N: int, K: int) -> int:
     """Workspace bytes of ``int2_fp16_upcvt_gemm`` (0 when none is needed)."""
     return lib().ternocl_int2_gemm_ws_bytes(M, N, K)
+
+
+def kw_tile_of(entry: int, bf16: bool, M: int, N: int, K: int, E: int = 0, ws_bytes: int = 0):
+    """(rows, cols, K waves, K slices, repacked) of the K-over-waves tile that a call takes, None where
+    another engine runs it (test hook; entry 0 int2, 1 s8 x s2, 2 M-tiled BITCOS, 3 MoE)."""
+    t = _abi.KwTile()
+    if not lib().ternocl_kw_tile_of(entry, BF16 if bf16 else FP16, M, N, K, E, ws_bytes, ctypes.byref(t)):
+        return None
+    return t.rows, t.cols, t.k_waves, t.k_slices, bool(t.repacked)
 
 
 def workspace_zero(ws, stream=None) -> None:

@@ -15,6 +15,11 @@ class GemvTile(C.Structure):
     _fields_ = [("engine", C.c_int), ("waves", C.c_int), ("cols_per_lane", C.c_int),
                 ("groups_per_wave", C.c_int), ("col_lanes", C.c_int), ("k_slices", C.c_int)]
 
+
+class KwTile(C.Structure):
+    """ternocl_kw_tile (include/ternocl_amd.h)."""
+    _fields_ = [("rows", C.c_int), ("cols", C.c_int), ("k_waves", C.c_int), ("k_slices", C.c_int), ("repacked", C.c_int)]
+
 I = C.c_int
 Z = C.c_size_t
 
@@ -24,6 +29,7 @@ SYMBOLS: dict[str, tuple] = {
     "ternocl_last_error": (C.c_char_p, []),
     "ternocl_version": (C.c_char_p, []),
     "ternocl_int2_gemm_ws_bytes": (Z, [I, I, I]),
+    "ternocl_kw_tile_of": (I, [I, I, I, I, I, I, Z, C.POINTER(KwTile)]),
     "ternocl_workspace_zero": (I, [P, Z, P]),
     "ternocl_int2_fp16_upcvt_gemm": (I, [I, P, P, P, P, P, P, I, I, I, I, I, P, Z, P]),
     "ternocl_int2_fp16_upcvt_gemm_ex": (I, [I, P, P, P, P, P, P, I, I, I, I, I, P, Z,

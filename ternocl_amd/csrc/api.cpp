@@ -69,6 +69,7 @@ size_t int2_gemm_ws_need(int M, int N, int K);
 ternocl_status int2_gemm_decode_run(int dtype, const uint32_t *B, uint32_t *D, int K, int N, hipStream_t st);
 // kernels (int2_gemm_kw.hip)
 size_t int2_gemm_kw_ws_need(int M, int N, int K);
+bool int2_gemm_kw_tile(int M, int N, int K, bool bf, size_t ws_bytes, bool force, ternocl_kw_tile &t);
 bool int2_gemm_kw_run(int dtype, const void *A, const uint32_t *B, const void *S, void *C, const void *Other,
                       const void *Bias, int M, int N, int K, int postop, int out_f32, hipStream_t st, void *ws,
                       size_t ws_bytes, bool force, ternocl_status &s);
@@ -80,7 +81,9 @@ ternocl_status int2_int8_gemm_run(int dtype, const void *A, const int8_t *Aq, co
                                   const void *Bias, int M, int N, int K, int postop, int out_f32,
                                   hipStream_t st, void *ws = nullptr, size_t ws_bytes = 0);
 ternocl_status int2_s8_decode_run(const uint32_t *B, uint32_t *D, int K, int N, hipStream_t st);
-size_t int2_int8_kw_ws_need(int M, int N, int K);  // int2_int8_kw.hip
+// kernels (int2_int8_kw.hip)
+size_t int2_int8_kw_ws_need(int M, int N, int K);
+bool int2_int8_kw_tile(int M, int N, int K, size_t ws_bytes, ternocl_kw_tile &t);
 // kernels (bitcos.hip)
 int bitcos_max_ls();
 int bitcos_pick_ls(int N, int K);
@@ -95,6 +98,7 @@ ternocl_status bitcos_gemm_mt_run(int dtype, const void *A, const uint32_t *Bc, 
 // kernels (bitcos_kw.hip): how a call of the M-tiled entry runs there (0: not)
 int bitcos_kw_auto(int M, int N, int K, bool bf, bool repack, const void *A, const void *Bc, const void *S, const void *C,
                    const void *Other, const void *Bias);
+bool bitcos_kw_tile(int M, int N, int K, bool bf, ternocl_kw_tile &t);
 ternocl_status bitcos_kw_run(int dtype, const void *A, const uint32_t *Bc, const void *S, void *C, const void *Other,
                              const void *Bias, int M, int N, int K, int postop, int out_f32, hipStream_t st);
 ternocl_status bitcos_slice_ranks_run(const uint32_t *Bc, uint32_t *SR, int N, int K, int ls,
@@ -111,6 +115,8 @@ ternocl_status bitcos_fwht_gemv_run(int dtype, const void *x, const int8_t *sign
                                     const uint32_t *SR, int ls, void *C, const void *Other, const void *Bias, int M,
                                     int N, int K, int postop, int out_f32, hipStream_t st, void *ws,
                                     size_t ws_bytes);  // bitcos.hip
+// kernels (moe_kw.hip)
+bool moe_kw_tile_of(int G, int E, int N, int K, ternocl_kw_tile &t);
 // kernels (moe.hip, int2_gemm_mfma.hip)
 int moe_tile_rows();
 ternocl_status moe_route_run(const int *ids, int *meta, int *perm, int *inv, int G, int E, hipStream_t st,
@@ -203,6 +209,18 @@ size_t ternocl_int2_gemm_ws_bytes(int M, int N, int K) {
     // the slice sums of the K-split engines' plans (an upper bound of the two)
     const size_t a = int2_gemm_ws_need(M, N, K), b = int2_gemm_kw_ws_need(M, N, K);
     return a > b ? a : b;
+}
+
+int ternocl_kw_tile_of(int entry, int dtype, int M, int N, int K, int E, size_t ws_bytes, ternocl_kw_tile *tile) {
+    ternocl_kw_tile t = {0, 0, 0, 0, 0};
+    const bool bf = dtype == TERNOCL_BF16, ok = M >= 1 && N >= 16 && N % 16 == 0 && K >= kGS && K % kGS == 0;
+    bool kw = false;
+    if (ok && entry == 0) kw = int2_gemm_kw_tile(M, N, K, bf, ws_bytes, false, t);
+    else if (ok && entry == 1) kw = int2_int8_kw_tile(M, N, K, ws_bytes, t);
+    else if (ok && entry == 2) kw = bitcos_kw_tile(M, N, K, bf, t);
+    else if (ok && entry == 3 && E >= 1) kw = moe_kw_tile_of(M, E, N, K, t);
+    if (tile) *tile = t;
+    return kw ? 1 : 0;
 }
 
 ternocl_status ternocl_workspace_zero(void *ws, size_t ws_bytes, void *stream) {

@@ -265,6 +265,18 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
 
+// (for ternocl_kw_tile_of: the tile of an M-tiled call on aligned operands; repacked:
+// the workspace form runs int2_gemm_kw_run on the re-packed words)
+bool bitcos_kw_tile(int M, int N, int K, bool bf, ternocl_kw_tile &t) {
+    int wk;
+    bool repacked;
+    double us;
+    if (!bckw_route(M, N, K, bf, wk, repacked)) return false;
+    const BcTile &b = kBcTiles[bckw_tile(M, N, K, wk, us)];
+    t = {b.bm, b.bn, b.wk, 1, repacked};
+    return true;
+}
+
 // How a call of the M-tiled entry runs here: 0 not, 1 bitcos_kw_run, 2 (repack:
 // the caller re-packs the weights) int2_gemm_kw_run on the re-packed words.
 int bitcos_kw_auto(int M, int N, int K, bool bf, bool repack, const void *A, const void *Bc, const void *S, const void *C,

@@ -185,6 +185,26 @@ size_t int2_gemm_kw_ws_need(int M, int N, int K) {
     return kWsHeader + (size_t)p.ks * M * N * 4;
 }
 
+// The tile and K slices of an automatic call on aligned operands with ws_bytes of
+// workspace (0: none), false where another engine runs it: the choice of
+// int2_gemm_kw_run, for ternocl_kw_tile_of.
+static bool kw_choose(int M, int N, int K, bool bf, size_t ws_bytes, bool force, KwPlan &p) {
+    bool split = ws_bytes > kWsHeader && M > 16;
+    p = kw_plan(M, N, K, split);
+    if (p.ks > 1 && ws_bytes < kWsHeader + (size_t)p.ks * M * N * 4) {
+        p = kw_plan(M, N, K, false);
+        split = false;
+    }
+    return force || kw_wins(p, M, N, K, split, bf);
+}
+
+bool int2_gemm_kw_tile(int M, int N, int K, bool bf, size_t ws_bytes, bool force, ternocl_kw_tile &t) {
+    KwPlan p;
+    if (M <= 8 || M > 2048 || !kw_choose(M, N, K, bf, ws_bytes, force, p)) return false;
+    t = {kKwTiles[p.tile].bm, kKwTiles[p.tile].bn, p.tile <= 1 ? 8 : 4, p.ks, 0};
+    return true;
+}
+
 // Runs the call here if this is its automatic engine (force: whichever the
 // models prefer) and returns whether it did; the status in s.  A K split needs
 // its slice sums in ws; with less the unsplit plan is weighed.  The vector
@@ -196,14 +216,8 @@ bool int2_gemm_kw_run(int dtype, const void *A, const uint32_t *B, const void *S
     if (M <= 8 || M > 2048 || !aligned16(A) || !aligned16(B) || !aligned16(S) || !aligned16(C) || !aligned16(Other) ||
         !aligned16(Bias))
         return false;
-    const bool ws_ok = ws && ws_bytes > kWsHeader && aligned16(ws) && M > 16;
-    KwPlan p = kw_plan(M, N, K, ws_ok);
-    bool split = ws_ok;
-    if (p.ks > 1 && ws_bytes < kWsHeader + (size_t)p.ks * M * N * 4) {
-        p = kw_plan(M, N, K, false);
-        split = false;
-    }
-    if (!force && !kw_wins(p, M, N, K, split, bf)) return false;
+    KwPlan p;
+    if (!kw_choose(M, N, K, bf, ws && aligned16(ws) ? ws_bytes : 0, force, p)) return false;
     uint32_t *cnt = p.ks > 1 ? (uint32_t *)ws : nullptr;
     float *part = p.ks > 1 ? (float *)((uint8_t *)ws + kWsHeader) : nullptr;
     auto go = [&](auto cfg) {

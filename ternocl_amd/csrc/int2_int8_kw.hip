@@ -305,6 +305,26 @@ size_t int2_int8_kw_ws_need(int M, int N, int K) {
     return p.ks > 1 && i8kw_wins(p, M, N, K, true) ? kWsHeader + (size_t)p.ks * M * N * 4 : 0;
 }
 
+// The tile and K slices of a call on aligned operands with ws_bytes of workspace
+// (0: none), false where the tile engines run it: the choice of int2_int8_kw_run,
+// for ternocl_kw_tile_of.
+static bool i8kw_choose(int M, int N, int K, size_t ws_bytes, I8Plan &p) {
+    bool split = ws_bytes > kWsHeader;
+    p = i8kw_plan(M, N, K, split);
+    if (p.ks > 1 && ws_bytes < kWsHeader + (size_t)p.ks * M * N * 4) {
+        p = i8kw_plan(M, N, K, false);
+        split = false;
+    }
+    return i8kw_wins(p, M, N, K, split);
+}
+
+bool int2_int8_kw_tile(int M, int N, int K, size_t ws_bytes, ternocl_kw_tile &t) {
+    I8Plan p;
+    if (M <= 4 || M > 2048 || !i8kw_choose(M, N, K, ws_bytes, p)) return false;
+    t = {kI8Tiles[p.tile].bm, kI8Tiles[p.tile].bn, p.tile <= 1 ? 8 : 4, p.ks, 0};
+    return true;
+}
+
 // Runs the call here if the models prefer this engine and returns whether it
 // did; the error in e.  Aq non-null: upfront mode, else A's DT rows; the choice
 // is the same in both, whose bits agree.  A K split needs its slice sums in ws;
@@ -316,13 +336,8 @@ bool int2_int8_kw_run(int dtype, const void *A, const int8_t *Aq, const void *SA
     if (M > 2048 || !aligned16(Aq ? (const void *)Aq : A) || !aligned16(B) || !aligned16(SB) || !aligned16(C) ||
         !aligned16(Other) || !aligned16(Bias))
         return false;
-    bool split = ws && ws_bytes > kWsHeader && aligned16(ws);
-    I8Plan p = i8kw_plan(M, N, K, split);
-    if (p.ks > 1 && ws_bytes < kWsHeader + (size_t)p.ks * M * N * 4) {
-        p = i8kw_plan(M, N, K, false);
-        split = false;
-    }
-    if (!i8kw_wins(p, M, N, K, split)) return false;
+    I8Plan p;
+    if (!i8kw_choose(M, N, K, ws && aligned16(ws) ? ws_bytes : 0, p)) return false;
     uint32_t *cnt = p.ks > 1 ? (uint32_t *)ws : nullptr;
     float *part = p.ks > 1 ? (float *)((uint8_t *)ws + kWsHeader) : nullptr;
     auto go = [&](auto cfg) {

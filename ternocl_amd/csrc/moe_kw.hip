@@ -125,6 +125,14 @@ static bool moe_kw_takes(int G, int E, int N, int K, bool &tall) {
     return (long)G <= 64L * E && (double)tiles * N * K <= 190e6;
 }
 
+// (for ternocl_kw_tile_of: the tile of one of the layer's products)
+bool moe_kw_tile_of(int G, int E, int N, int K, ternocl_kw_tile &t) {
+    bool tall;
+    if (!moe_kw_takes(G, E, N, K, tall)) return false;
+    t = {tall ? 64 : 32, 64, 4, 1, 0};
+    return true;
+}
+
 // The grouped GEMM (B2 non-null: up and gate in one launch) where the rule above
 // takes it and the operands are 16-byte aligned; returns whether it ran.
 bool moe_gemm_kw_run(int dtype, const int *meta, const void *A, const int *perm, int topk, const uint32_t *B, const void *S,
