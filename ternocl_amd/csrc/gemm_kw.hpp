@@ -241,18 +241,45 @@ __device__ __forceinline__ void kw_store(void *C, const uint16_t *Other, const v
 }
 
 
+// A slice's arrival at its tile's counter (lane 0's atomics, broadcast): the
+// arrivals before this one.  The counter reads 0 between calls and kKwLive + n
+// after n of ksn arrivals; anything else is left from another use of the
+// workspace's memory (these calls' earlier engines took a workspace that nothing
+// had zeroed) and counts as 0.  The last arrival stores 0.  An exchange fails only
+// where another slice arrived meanwhile (or on the first guess of 0), so at most
+// ksn times; the last arrival, on the critical path, makes one failing exchange,
+// as long as an increment.
+constexpr uint64_t kKwLive = 0x9E6D3A5171C3B200ull;
+__device__ __forceinline__ uint32_t kw_arrive(uint64_t *c, int ksn, int lane) {
+    uint32_t prev = 0;
+    if (lane == 0) {
+        uint64_t seen = 0;
+        while (true) {
+            prev = seen - kKwLive < (uint64_t)ksn ? (uint32_t)(seen - kKwLive) : 0u;
+            if (prev == (uint32_t)(ksn - 1)) {
+                __hip_atomic_store(c, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+            }
+            if (__hip_atomic_compare_exchange_strong(c, &seen, kKwLive + prev + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT))
+                break;
+        }
+    }
+    return __builtin_amdgcn_readfirstlane(prev);
+}
+
 // The sums of the waves' K parts in wave order (through LDS, a round of row
 // blocks at a time), then the epilogue of the tile's rows [0, mrows) (C rows from
 // m0) and columns [n0, n0 + 32 CB) (below N).  ksn > 1: slice sl's sums go to part
 // [ksn][M][N] (agent-scope stores), and the last of the tile's ksn workgroups
-// (its counter cnt, split_arrive) adds the slices in order -- the handoff of the
+// (its counter cnt, kw_arrive) adds the slices in order -- the handoff of the
 // decode GEMV's K split (int2_gemv_f4.hip).  DUAL (KwDual's sums, ksn == 1): C =
 // DT(silu(gate) * DT(up)) on CB / 2 columns a lane, the bits of the up product
 // stored in DT and read by the gate product's epilogue.
 template <class Cfg, bool BF16, bool DUAL = false>
 __device__ __forceinline__ void kw_finish(f32x16_t acc[Cfg::MB][Cfg::CB], uint8_t *lds, void *C, const uint16_t *Other,
                                           const void *Bias, int M, int N, int m0, int mrows, int n0, int postop, int out_f32,
-                                          int ksn, int sl, float *part, uint32_t *cnt) {
+                                          int ksn, int sl, float *part, uint64_t *cnt) {
     constexpr int MB = Cfg::MB, CB = Cfg::CB, WK = Cfg::WK, CS = DUAL ? CB / 2 : CB;
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, q = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kw = wave / Cfg::WM, wm = wave % Cfg::WM;
@@ -350,7 +377,7 @@ __device__ __forceinline__ void kw_finish(f32x16_t acc[Cfg::MB][Cfg::CB], uint8_
     __syncthreads();  // every wave's sums are stored
     uint32_t *flag = (uint32_t *)lds;
     if (wave == 0) {
-        const uint32_t prev = split_arrive(cnt, ksn, lane);
+        const uint32_t prev = kw_arrive(cnt, ksn, lane);
         if (lane == 0) *flag = prev;
     }
     __syncthreads();

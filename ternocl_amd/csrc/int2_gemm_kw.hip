@@ -51,7 +51,7 @@ template <class Cfg, bool BF16>
 __global__ void __launch_bounds__(Cfg::THREADS)
 k_int2_gemm_kw(const uint16_t *__restrict__ A, const uint32_t *__restrict__ B, const uint16_t *__restrict__ S,
                void *__restrict__ C, const uint16_t *__restrict__ Other, const void *__restrict__ Bias, int M, int N,
-               int K, int postop, int out_f32, int ksn, float *part, uint32_t *cnt) {
+               int K, int postop, int out_f32, int ksn, float *part, uint64_t *cnt) {
     constexpr int MB = Cfg::MB, CB = Cfg::CB, WK = Cfg::WK;
     extern __shared__ __attribute__((aligned(16))) uint8_t kw_lds[];
     const int mt = (M + Cfg::BM - 1) / Cfg::BM, nt = (N + Cfg::BN - 1) / Cfg::BN;
@@ -88,7 +88,7 @@ k_int2_gemm_kw(const uint16_t *__restrict__ A, const uint32_t *__restrict__ B, c
 
 template <class Cfg, bool BF16>
 hipError_t kw_launch(const void *A, const uint32_t *B, const void *S, void *C, const void *Other, const void *Bias, int M,
-                     int N, int K, int postop, int out_f32, int ksn, float *part, uint32_t *cnt, hipStream_t st) {
+                     int N, int K, int postop, int out_f32, int ksn, float *part, uint64_t *cnt, hipStream_t st) {
     const int mt = (M + Cfg::BM - 1) / Cfg::BM, nt = (N + Cfg::BN - 1) / Cfg::BN;
     hipLaunchKernelGGL((k_int2_gemm_kw<Cfg, BF16>), dim3(xcd_ashare_grid(mt * ksn, nt)), dim3(Cfg::THREADS),
                        Cfg::LDS_BYTES, st, (const uint16_t *)A, B, (const uint16_t *)S, C, (const uint16_t *)Other, Bias,
@@ -128,7 +128,7 @@ KwPlan kw_plan(int M, int N, int K, bool split) {
         if (t.bm > 32 && t.bm >= 2 * M) continue;  // half the tile's rows idle: a lower one does it
         const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
         for (int ks = 1; ks <= 8; ++ks) {
-            if (ks > 1 && (!split || K / ks < 512 || tiles * ks > 1024 || tiles * 4 > (long)kWsHeader)) break;
+            if (ks > 1 && (!split || K / ks < 512 || tiles * ks > 1024 || tiles * 8 > (long)kWsHeader)) break;
             const double rounds = (double)((tiles * ks + 255) / 256);
             double us = t.base * (0.5 + 0.5 * rounds) + t.slope * rounds * K / (1024.0 * ks);
             if (ks > 1) us += 1.2 + 8e-6 * ks * M * N / 4.0;
@@ -218,7 +218,7 @@ bool int2_gemm_kw_run(int dtype, const void *A, const uint32_t *B, const void *S
         return false;
     KwPlan p;
     if (!kw_choose(M, N, K, bf, ws && aligned16(ws) ? ws_bytes : 0, force, p)) return false;
-    uint32_t *cnt = p.ks > 1 ? (uint32_t *)ws : nullptr;
+    uint64_t *cnt = p.ks > 1 ? (uint64_t *)ws : nullptr;
     float *part = p.ks > 1 ? (float *)((uint8_t *)ws + kWsHeader) : nullptr;
     auto go = [&](auto cfg) {
         typedef decltype(cfg) Cfg;

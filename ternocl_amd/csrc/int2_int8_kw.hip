@@ -36,7 +36,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
 k_int2_int8_kw(const void *__restrict__ Asrc, const uint16_t *__restrict__ SA, const uint32_t *__restrict__ B,
                const uint16_t *__restrict__ SB, void *__restrict__ C, const uint16_t *__restrict__ Other,
                const void *__restrict__ Bias, int M, int N, int K, int postop, int out_f32, int ksn, float *part,
-               uint32_t *cnt) {
+               uint64_t *cnt) {
     constexpr int MB = Cfg::MB, CB = Cfg::CB, WK = Cfg::WK, PF = Cfg::PF;
     static_assert(MB <= 2, "a lane per row for 1 / SA");
     extern __shared__ __attribute__((aligned(16))) uint8_t kw_lds[];
@@ -215,7 +215,7 @@ template <class Cfg> constexpr int i8kw_lds() {
 
 template <class Cfg, bool BF16, bool QA>
 hipError_t i8kw_launch(const void *A, const void *SA, const uint32_t *B, const void *SB, void *C, const void *Other,
-                       const void *Bias, int M, int N, int K, int postop, int out_f32, int ksn, float *part, uint32_t *cnt,
+                       const void *Bias, int M, int N, int K, int postop, int out_f32, int ksn, float *part, uint64_t *cnt,
                        hipStream_t st) {
     const int mt = (M + Cfg::BM - 1) / Cfg::BM, nt = (N + Cfg::BN - 1) / Cfg::BN;
     hipLaunchKernelGGL((k_int2_int8_kw<Cfg, BF16, QA>), dim3(xcd_ashare_grid(mt * ksn, nt)), dim3(Cfg::THREADS),
@@ -265,7 +265,7 @@ I8Plan i8kw_plan(int M, int N, int K, bool split) {
         if (t.bm > 32 && t.bm >= 2 * M) continue;  // half the tile's rows idle
         const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
         for (int ks = 1; ks <= 8; ++ks) {
-            if (ks > 1 && (!split || K / ks < 512 || tiles * ks > 1024 || tiles * 4 > (long)kWsHeader)) break;
+            if (ks > 1 && (!split || K / ks < 512 || tiles * ks > 1024 || tiles * 8 > (long)kWsHeader)) break;
             double us = i8kw_us(i, (double)tiles * ks, K / (1024.0 * ks));
             if (ks > 1) us += 1.2 + 8e-6 * ks * M * N / 4.0;
             if (us < best.us - 1e-9) best = {i, ks, us};
@@ -338,7 +338,7 @@ bool int2_int8_kw_run(int dtype, const void *A, const int8_t *Aq, const void *SA
         return false;
     I8Plan p;
     if (!i8kw_choose(M, N, K, ws && aligned16(ws) ? ws_bytes : 0, p)) return false;
-    uint32_t *cnt = p.ks > 1 ? (uint32_t *)ws : nullptr;
+    uint64_t *cnt = p.ks > 1 ? (uint64_t *)ws : nullptr;
     float *part = p.ks > 1 ? (float *)((uint8_t *)ws + kWsHeader) : nullptr;
     auto go = [&](auto cfg) {
         typedef decltype(cfg) Cfg;

@@ -245,3 +245,35 @@ def test_split_gemvs_on_a_workspace_never_zeroed(dev, bf16):
     wsb = torch.full((needb,), 0x7f, dtype=torch.uint8, device="cuda")
     assert np.array_equal(gemvb(wsb), wantb), "BITCOS GEMV on an unzeroed workspace differs"
     assert _counters_reset(wsb), "BITCOS GEMV counters not reset"
+
+
+@pytest.mark.parametrize("fill", [1, 2, 0x7f7f7f7f])
+@pytest.mark.parametrize("M,K,N", [(48, 14336, 4096), (130, 8192, 528)])
+def test_k_slices_on_a_workspace_from_other_use(dev, M, K, N, fill):
+    """The K slices of calls of more than 16 rows (int8: more than 4) need no zeroed workspace, as
+    before they had counters: words that could pass for a count of arrivals (1, 2: the memory held
+    indices, say) give the bits of a zeroed workspace, and the words used are left at zero."""
+    import torch
+    import ternocl_amd as T
+    A, B, S, _, _ = _int2_operands(13, M, K, N, True)
+    SA = torch.zeros((K // 128, T.ldsa(M)), dtype=A.dtype, device="cuda")
+    Aq = torch.zeros((M, K), dtype=torch.int8, device="cuda")
+    T.quant_a(A, SA, Aq, M, K)
+
+    def call(entry, word):
+        need = (T.int2_int8_gemm_ws_bytes if entry else T.int2_gemm_ws_bytes)(M, N, K)
+        assert T.kw_tile_of(entry, True, M, N, K, ws_bytes=need)[3] > 1, "no K slices"
+        ws = torch.full((need // 4,), word, dtype=torch.int32, device="cuda")
+        C = torch.zeros((M, N), dtype=A.dtype, device="cuda")
+        if entry:
+            T.int2_int8_gemm(None, Aq, SA, B, S, C, None, None, M, N, K, ws=ws)
+        else:
+            T.int2_fp16_upcvt_gemm(A, B, S, C, None, None, M, N, K, ws=ws)
+        torch.cuda.synchronize()
+        return host_u16(C), ws[:T.WS_HEADER_BYTES // 4].cpu().numpy().view(np.uint32)
+    for entry in (0, 1):
+        print(f"K slices on used memory entry={entry} M={M} K={K} N={N} fill={fill:#x}", flush=True)
+        want, _ = call(entry, 0)
+        got, header = call(entry, fill)
+        assert np.array_equal(got, want), "other bits than on a zeroed workspace"
+        assert np.isin(header, (0, fill)).all() and (header == 0).any(), "a counter was left set"
