@@ -938,7 +938,7 @@ int moe_tile_rows() { return kMoeTileRows; }
 
 // Column tile of the MoE GEMMs: the widest of 512 / 256 / 128 columns whose
 // ragged last tile idles at most 1/10 of the MFMA work.
-static int moe_bn(int N, int widest) {
+int moe_bn(int N, int widest) {
     for (int bn = widest; bn > 128; bn >>= 1)
         if ((long)((N + bn - 1) / bn) * bn * 10 <= (long)N * 11) return bn;
     return 128;

@@ -5,15 +5,17 @@
 //
 // With a few rows an expert (T = 16, 128 experts, top-8: one or two) the 128-row
 // tiles stage and multiply mostly nothing and walk K stage by stage behind a
-// barrier: ~32 us a GEMM whatever T is.  Here a workgroup of four waves takes 32
-// (or 64) of an expert's rows and a strip of its columns, each wave a quarter of K.
+// barrier: ~32 us a GEMM whatever T is.  Here a workgroup of four waves takes 32 of
+// an expert's rows and a strip of its columns, each wave a quarter of K.
 // It finds its expert from the route's row offsets (a count and a scan over the
 // experts, 64 a step), so the route and its tile list stay as they are.
 #include "gemm_kw.hpp"
 
 #include <algorithm>
+#include <cmath>
 
 namespace tcl {
+int moe_bn(int N, int widest);  // int2_gemm_mfma.hip
 namespace {
 
 // The expert and the first row (within it) of row tile `tile`, tiles of bm rows
@@ -107,29 +109,63 @@ void moe_kw_launch(const int *meta, const void *A, const int *perm, int topk, co
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
+// ---- host side: where this engine runs -------------------------------------------
+
+// The times (us) of a whole layer with H x I experts (up and gate in one launch,
+// K = H; down, K = I) on these tiles and on the 128-row ones, fitted to
+// graph-timed layers of 20912 random sizes (both types; E = 8..256, H = 512..4096, I =
+// 256..3072, up to 64 rows an expert, even to skewed routings): 5..95% of them
+// within 0.84..1.16 and 0.80..1.15 of the fit.  rows per expert are taken as
+// Poisson: E (1 - e^-l) experts with rows, l = G / E.
+//   * here: a launch cannot be shorter than its waves' walk (by K), and a workgroup
+//     costs its part of the decode (by K) and a fixed start and end; 64 columns x 32
+//     rows a workgroup, past ~20 rows an expert some experts take a second tile;
+//   * the 128-row tiles: K stages of constant length, dearer once the tiles (two
+//     experts' rows share one, up to 64 each) pass one a CU.
+struct MoeUs {
+    double kw, tile;
+};
+MoeUs moe_layer_us(int G, int E, int H, int I) {
+    const double l = (double)G / E, with = E * (1.0 - std::exp(-l)), h = H / 1024.0, i = I / 1024.0;
+    const double t = l > 20.0 ? std::max(with, E * (l / 32.0 + 0.45)) : with, p = std::max(with / 2.0, 1.0);
+    auto up_to = [](int n, int b) { return (double)((n + b - 1) / b); };
+    const double wu = t * up_to(I, 64) / 256.0, wd = t * up_to(H, 64) / 256.0;
+    const int bu = moe_bn(I, 256), bd = moe_bn(H, 512);
+    const double ru = p * up_to(I, bu) / 256.0, rd = p * up_to(H, bd) / 256.0;
+    MoeUs us;
+    us.kw = 18.5 + std::hypot(2.5 * h, (3.25 * h + 2.35) * wu) + std::hypot(1.2 * i, (0.65 * i + 1.2) * wd);
+    us.tile = 20.7 + (bu == 256 ? 17.8 : 9.9) * h * (1.0 + std::min(ru, 1.0) + 2.5 * std::max(ru - 1.0, 0.0)) +
+              (bd == 512 ? 18.6 : bd == 256 ? 10.0 : 6.4) * i * (1.0 - 0.15 * std::min(rd, 1.0) + 1.6 * std::max(rd - 1.0, 0.0));
+    return us;
+}
+
 }  // namespace
 
-// Whether G rows over E experts of K x N weights run here: at most 64 rows an
-// expert on average, and weights to decode (of the experts some row takes, once
-// per row tile) below 190 M a matrix -- a rule on sizes that the three GEMMs of a
-// layer and the single grouped GEMM share, so their bits agree.  Measured layers
-// (bf16, top-8 unless said, graph-timed, us; 128-row tiles -> these): E = 128 H = 2048
-// I = 768, T = 1 76 -> 29, T = 8 79 -> 52, T = 16 81 -> 67, past the line T = 64 84
-// against 92; E = 64 I = 1408, T = 16 91 -> 80, T = 128 94 -> 84, past it T = 256
-// 113 against 140; E = 16 top-4, H = 1024 I = 512, T = 40 49 -> 22, H = 3072 I =
-// 1536, T = 128 (64-row tiles) 130 -> 68.  What bounds the larger ones is the
-// decode's VALU work: ~26 instructions per 16 weights against one tile's rows.
-static bool moe_kw_takes(int G, int E, int N, int K, bool &tall) {
-    tall = (long)G > 24L * E;
-    const long tiles = std::max<long>(std::min(E, G), G / (tall ? 64 : 32));
-    return (long)G <= 64L * E && (double)tiles * N * K <= 190e6;
+// Whether G rows over E experts of K x N weights run here.  A layer's products (K x
+// N and N x K) and the single grouped GEMM ask alike, so their bits agree: a
+// product does not know which of the two sizes is the layer's H: the layer with the
+// larger one as H, the usual one, counts twice, the other once.  Ahead by more than
+// the fits' spread: of the 20912 layers 78% run here and 13 lose more than 3%, two
+// of them more than 10% (a bound on the weights decoded, with a row tile an expert,
+// lost more than 3% in 1558, up to 2.5x).  Measured layers (bf16,
+// top-8 unless said, us; 128-row tiles / here): E = 128 H = 2048 I = 768, T = 1 77 /
+// 30, T = 8 78 / 50, T = 16 80 / 67, not taken T = 32 83 / 85, T = 64 85 / 92; E = 64
+// I = 1408, T = 16 92 / 71, T = 64 93 / 81, T = 128 97 / 84, not taken T = 256 115 /
+// 111, T = 512 171 / 171; E = 16 top-4, H = 1024 I = 512, T = 40 50 / 24, H = 3072 I =
+// 1536, T = 128 122 / 61.  64-row tiles were faster than these 32-row ones by more
+// than 3% in 9 of the layers taken (E = 64 I = 1408, T = 128 139; E = 16 H = 3072, T
+// = 128 69).
+static bool moe_kw_takes(int G, int E, int N, int K) {
+    if ((long)G > 64L * E) return false;
+    const int large = std::max(N, K), small = std::min(N, K);
+    const MoeUs a = moe_layer_us(G, E, large, small), b = moe_layer_us(G, E, small, large);
+    return 2.0 * a.kw + b.kw < 0.89 * (2.0 * a.tile + b.tile);
 }
 
 // (for ternocl_kw_tile_of: the tile of one of the layer's products)
 bool moe_kw_tile_of(int G, int E, int N, int K, ternocl_kw_tile &t) {
-    bool tall;
-    if (!moe_kw_takes(G, E, N, K, tall)) return false;
-    t = {tall ? 64 : 32, 64, 4, 1, 0};
+    if (!moe_kw_takes(G, E, N, K)) return false;
+    t = {32, 64, 4, 1, 0};
     return true;
 }
 
@@ -138,16 +174,13 @@ bool moe_kw_tile_of(int G, int E, int N, int K, ternocl_kw_tile &t) {
 bool moe_gemm_kw_run(int dtype, const int *meta, const void *A, const int *perm, int topk, const uint32_t *B, const void *S,
                      const uint32_t *B2, const void *S2, void *C, const void *Other, int E, int G, int N, int K, int postop,
                      int out_f32, hipStream_t st, ternocl_status &s) {
-    bool tall;
-    if (!moe_kw_takes(G, E, N, K, tall) || !aligned16(A) || !aligned16(B) || !aligned16(S) || !aligned16(B2) || !aligned16(S2) ||
+    if (!moe_kw_takes(G, E, N, K) || !aligned16(A) || !aligned16(B) || !aligned16(S) || !aligned16(B2) || !aligned16(S2) ||
         !aligned16(C) || !aligned16(Other))
         return false;
     auto go = [&](auto bf, auto dual) {
         constexpr bool BF = decltype(bf)::value, D = decltype(dual)::value;
-        typedef KwCfg<1, D ? 4 : 2, 1, 4, 2> Low;
-        typedef KwCfg<2, D ? 4 : 2, 1, 4, 2> Tall;
-        if (tall) moe_kw_launch<Tall, BF, D>(meta, A, perm, topk, B, S, B2, S2, C, Other, E, G, N, K, postop, out_f32, st);
-        else moe_kw_launch<Low, BF, D>(meta, A, perm, topk, B, S, B2, S2, C, Other, E, G, N, K, postop, out_f32, st);
+        moe_kw_launch<KwCfg<1, D ? 4 : 2, 1, 4, 2>, BF, D>(meta, A, perm, topk, B, S, B2, S2, C, Other, E, G, N, K, postop,
+                                                           out_f32, st);
     };
     if (dtype == TERNOCL_BF16) B2 ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
     else B2 ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
