@@ -10,15 +10,16 @@
 // word, the ranks meet in LDS), then walk it: a word costs ~30 instructions more
 // than the packed format's, once per row tile.  Measured (fp16, z = .5,
 // graph-timed, us; with the re-pack workspace / without -> this): K = N = 4096, M =
-// 16 51.5 / 70.2 -> 12.1, M = 128 51.8 / 71.6 -> 17.3, M = 256 53.9 / 71.9 -> 24.9; K =
-// 5376 N = 21504, M = 32 71.1 / 91.3 -> 31.8, M = 64 71.0 / 91.1 -> 44.6.  What
-// bounds it is the decode: ~24 instructions and four table reads per 16 rows.
+// 16 52.9 / 71.9 -> 13.2, M = 128 52.3 / 72.2 -> 17.7, M = 256 53.6 / 71.9 -> 24.2; K = N =
+// 5120, M = 128 62.8 / 89.9 -> 26.9; K = 5376 N = 21504, M = 32 74.2 / 95.5 -> 33.2, M =
+// 64 74.3 / 95.5 -> 46.5.  What bounds it is the decode: ~24 instructions and four table reads per 16 rows.
 #include "gemm_kw.hpp"
 
 #include <algorithm>
 
 namespace tcl {
-void int2_gemm_kw_model(int M, int N, int K, bool bf, double &kw_us, double &other_us, int &wk);  // int2_gemm_kw.hip
+// (int2_gemm_kw.hip)
+void int2_gemm_kw_model(int M, int N, int K, bool bf, double &kw_us, double &other_us, int &wk, bool &square);
 namespace {
 
 // BITCOS weights as the walk's B source (gemm_kw.hpp): per unit of 64 rows the
@@ -206,23 +207,25 @@ hipError_t bckw_launch(const void *A, const uint32_t *Bc, const void *S, void *C
 
 // ---- host side: tile choice ----------------------------------------------------
 
-// The compiled tiles (rows, columns, waves over K) and their launches' times (us,
-// k in 1024 rows), fitted to graph-timed runs (fp16, z = .5) over M = 4..512, K =
-// 1024..5376, N = 2048..21504: 32 x 32 and 64 x 32 and 64 x 64 with eight waves, 64
-// x 64 with four (two workgroups a CU).
+// The compiled tiles (rows, columns, waves over K) and their launches' times: once +
+// round R + (once_k + round_k R) k us for R rounds of 256 workgroups (a last one of
+// few costs a whole one; the 64 x 64 tile of four waves and the 32 x 32 one, two a
+// CU, less), k in 1024 rows.  Fitted to 15754 graph-timed sizes (both types, z = .3,
+// .5, .7, M = 9..1024, K = 128..14336, N = 16..34816), within 6% for 5..95% of each
+// round's.  A fit linear in the workgroups took a tile at 1.2 rounds for 1.2 times
+// one round's time: M = 459 K = 768 N = 2400 19.6 us against the re-pack and the
+// 128-row tiles' 17.6, M = 54 K = 896 N = 33376 29.2 against 21.9 for those decoding
+// in place.
 struct BcTile {
     int bm, bn, wk;
+    double once, round, once_k, round_k;
 };
-constexpr BcTile kBcTiles[] = {{32, 32, 8}, {64, 32, 8}, {64, 64, 8}, {64, 64, 4}};
+constexpr BcTile kBcTiles[] = {{32, 32, 8, 4.5, 1.6, 0.6, 1.28}, {64, 32, 8, 3.3, 3.95, 0.2, 2.2},
+                               {64, 64, 8, 3.4, 5.4, 0.3, 3.45}, {64, 64, 4, 5.3, 2.2, 1.5, 3.05}};
 
-double bckw_us(int tile, double wgs, double k) {
-    const double r = wgs / 256.0;
-    switch (tile) {
-    case 0: return r <= 1 ? 4.8 + 2.1 * k : 6.0 + 1.78 * k * r;
-    case 1: return r <= 1 ? 6.0 + 2.85 * k : 6.0 + 3.3 * k * r;
-    case 2: return 7.0 + (r <= 1 ? 4.4 * k : 4.6 * k * r);
-    default: return r <= 1 ? 6.0 + 5.1 * k : r <= 2 ? 8.0 + 7.2 * k : 8.0 + 4.1 * k * r;
-    }
+double bckw_us(const BcTile &t, long wgs, double k) {
+    const double r = (double)((wgs + 255) / 256);
+    return t.once + t.round * r + (t.once_k + t.round_k * r) * k;
 }
 
 // The cheapest tile with wk waves over K (0: any).
@@ -232,7 +235,7 @@ int bckw_tile(int M, int N, int K, int wk, double &us) {
     for (int i = 0; i < 4; ++i) {
         const BcTile &t = kBcTiles[i];
         if ((wk && t.wk != wk) || (wk == 0 && t.bm > 32 && t.bm >= 2 * M)) continue;
-        const double u = bckw_us(i, (double)((long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn)), K / 1024.0);
+        const double u = bckw_us(t, (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn), K / 1024.0);
         if (u < us) {
             us = u;
             best = i;
@@ -250,15 +253,17 @@ bool bckw_route(int M, int N, int K, bool bf, int &wk, bool &repacked) {
     if (M <= 8 || M > 1024) return false;
     double direct, kw, other, chosen;
     int kwk;
+    bool square;
     const int t = bckw_tile(M, N, K, 0, direct);
-    int2_gemm_kw_model(M, N, K, bf, kw, other, kwk);
+    int2_gemm_kw_model(M, N, K, bf, kw, other, kwk, square);
     const double repack = 6.0 + 0.75 * K / 1024.0 + 5.5e-8 * K * N;  // k_bitcos_to_int2
     repacked = repack + kw < direct;
     wk = repacked ? kwk : kBcTiles[t].wk;
     bckw_tile(M, N, K, wk, chosen);
     // ahead (by more than the fits' spread) of the re-pack and the 128-row tiles, and
-    // without the workspace of the tiles that decode in place (1.2 - 1.75x the int2 ones)
-    return std::min(direct, repack + kw) < 0.95 * (repack + other) && chosen < 0.95 * 1.2 * other;
+    // without the workspace of the tiles that decode in place: 1.7 - 1.9x the int2 ones
+    // on 128 x 128, 1.15 - 1.3x on the wider
+    return std::min(direct, repack + kw) < 0.95 * (repack + other) && chosen < 0.95 * (square ? 1.5 : 1.2) * other;
 }
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }

@@ -43,6 +43,7 @@
 namespace tcl {
 // (int2_gemm_mfma.hip)
 bool gemm_half_tile(int M, int N);
+bool gemm_tile_is_square(int M, int N);
 int gemm_splits(int M, int N, int K);
 namespace {
 
@@ -162,12 +163,14 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 }  // namespace
 
 // The times the two models give a call without a K split (the M-tiled BITCOS
-// GEMM's choice, bitcos_kw.hip); wk: the waves over K of this engine's tile.
-void int2_gemm_kw_model(int M, int N, int K, bool bf, double &kw_us, double &other_us, int &wk) {
+// GEMM's choice, bitcos_kw.hip); wk: the waves over K of this engine's tile; square:
+// whether the other runs 128 x 128 tiles.
+void int2_gemm_kw_model(int M, int N, int K, bool bf, double &kw_us, double &other_us, int &wk, bool &square) {
     const KwPlan p = kw_plan(M, N, K, false);
     kw_us = p.us;
     other_us = kw_other_us(M, N, K, false, bf);
     wk = p.tile <= 1 ? 8 : 4;
+    square = gemm_tile_is_square(M, N);
 }
 
 // Whether plan p is the automatic engine of a call of M > 8 rows: always up to 16

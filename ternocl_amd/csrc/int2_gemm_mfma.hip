@@ -934,6 +934,9 @@ ternocl_status bitcos_gemm_mt_run(int dtype, const void *A, const uint32_t *Bc, 
     return check_launch();
 }
 
+// (the M-tiled BITCOS GEMM's engine choice)
+bool gemm_tile_is_square(int M, int N) { return gemm_plan(M, N).nmb == 4; }
+
 int moe_tile_rows() { return kMoeTileRows; }
 
 // Column tile of the MoE GEMMs: the widest of 512 / 256 / 128 columns whose

@@ -27,3 +27,24 @@ def test_moe_engine(Tk, E, topk, H, I, taken):
     import ternocl_amd as T
     up, down = (T.kw_tile_of(3, True, Tk * topk, N, K, E) for N, K in ((I, H), (H, I)))
     assert (up is not None) == taken and (down is not None) == taken
+
+
+# (M, K, N, tile or None): the M-tiled BITCOS GEMM.  A last round of a few workgroups costs a whole
+# one: the tile of 64 x 64 and eight waves these calls took at 1.1 to 2.1 rounds, against the tiles
+# that decode in place (no workspace) / the re-pack and the int2 ones
+BITCOS = [
+    (40, 256, 33968, None),              # 21.2 / 11.1 in place / 15.6 re-packed
+    (45, 640, 33952, None),              # 28.2 / 17.6 / 25.4
+    (10, 128, 33584, None),              # 32 x 32: 13.3 / 8.3 / 11.7
+    (102, 640, 10432, None),             # 20.2 / 17.3 / 19.7
+    (459, 768, 2400, None),              # 19.6 / 18.6 / 17.6
+    (32, 4096, 4096, (32, 32, 8)),       # 12.1 / 70 / 52
+]
+
+
+@pytest.mark.parametrize("M,K,N,tile", BITCOS)
+def test_bitcos_engine(M, K, N, tile):
+    import ternocl_amd as T
+    for bf16 in (False, True):
+        got = T.kw_tile_of(2, bf16, M, N, K)
+        assert (got[:3] if got else None) == tile
