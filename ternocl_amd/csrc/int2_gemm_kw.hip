@@ -84,7 +84,7 @@ k_int2_gemm_kw(const uint16_t *__restrict__ A, const uint32_t *__restrict__ B, c
         for (int cb = 0; cb < CB; ++cb) acc[mb][cb] = f32x16_t{};
     kw_walk<Cfg, BF16>(kw_lds + wave * (MB * 8192), A + (size_t)m0 * K, va, u0, u1, units, bs, acc);
     kw_finish<Cfg, BF16>(acc, kw_lds, C, Other, Bias, M, N, m0, mrows, n0, postop, out_f32, ksn, sl, part,
-                         ksn > 1 ? cnt + (size_t)tm * nt + tn : nullptr);
+                         ksn > 1 ? cnt + 2 * ((size_t)tm * nt + tn) : nullptr);
 }
 
 template <class Cfg, bool BF16>
@@ -129,7 +129,7 @@ KwPlan kw_plan(int M, int N, int K, bool split) {
         if (t.bm > 32 && t.bm >= 2 * M) continue;  // half the tile's rows idle: a lower one does it
         const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
         for (int ks = 1; ks <= 8; ++ks) {
-            if (ks > 1 && (!split || K / ks < 512 || tiles * ks > 1024 || tiles * 8 > (long)kWsHeader)) break;
+            if (ks > 1 && (!split || K / ks < 512 || tiles * ks > 1024 || tiles * 16 > (long)kWsHeader)) break;
             const double rounds = (double)((tiles * ks + 255) / 256);
             double us = t.base * (0.5 + 0.5 * rounds) + t.slope * rounds * K / (1024.0 * ks);
             if (ks > 1) us += 1.2 + 8e-6 * ks * M * N / 4.0;

@@ -205,7 +205,7 @@ k_int2_int8_kw(const void *__restrict__ Asrc, const uint16_t *__restrict__ SA, c
         }
     }
     kw_finish<Cfg, BF16>(acc, kw_lds, C, Other, Bias, M, N, m0, mrows, n0, postop, out_f32, ksn, sl, part,
-                         ksn > 1 ? cnt + (size_t)tm * nt + tn : nullptr);
+                         ksn > 1 ? cnt + 2 * ((size_t)tm * nt + tn) : nullptr);
 }
 
 template <class Cfg> constexpr int i8kw_lds() {
@@ -265,7 +265,7 @@ I8Plan i8kw_plan(int M, int N, int K, bool split) {
         if (t.bm > 32 && t.bm >= 2 * M) continue;  // half the tile's rows idle
         const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
         for (int ks = 1; ks <= 8; ++ks) {
-            if (ks > 1 && (!split || K / ks < 512 || tiles * ks > 1024 || tiles * 8 > (long)kWsHeader)) break;
+            if (ks > 1 && (!split || K / ks < 512 || tiles * ks > 1024 || tiles * 16 > (long)kWsHeader)) break;
             double us = i8kw_us(i, (double)tiles * ks, K / (1024.0 * ks));
             if (ks > 1) us += 1.2 + 8e-6 * ks * M * N / 4.0;
             if (us < best.us - 1e-9) best = {i, ks, us};
