@@ -147,7 +147,7 @@ typedef struct {
     int k_slices;   /* workgroups over K (> 1: sums in the workspace) */
     int repacked;   /* entry 2: with a workspace the weights are re-packed first */
 } ternocl_kw_tile;
-int ternocl_kw_tile_of(int entry, int dtype, int M, int N, int K, int E, size_t ws_bytes, ternocl_kw_tile *tile);
+int ternocl_kw_tile_of(int entry, int M, int N, int K, int E, size_t ws_bytes, ternocl_kw_tile *tile);
 
 /* Zero-fill device memory with a fill kernel (no hipMemset: graph-capturable). */
 ternocl_status ternocl_workspace_zero(void *ws, size_t ws_bytes, void *stream);

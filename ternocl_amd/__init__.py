@@ -118,11 +118,11 @@ def int2_gemm_ws_bytes(M: int, N: int, K: int) -> int:
     return lib().ternocl_int2_gemm_ws_bytes(M, N, K)
 
 
-def kw_tile_of(entry: int, bf16: bool, M: int, N: int, K: int, E: int = 0, ws_bytes: int = 0):
+def kw_tile_of(entry: int, M: int, N: int, K: int, E: int = 0, ws_bytes: int = 0):
     """(rows, cols, K waves, K slices, repacked) of the K-over-waves tile that a call takes, None where
     another engine runs it (test hook; entry 0 int2, 1 s8 x s2, 2 M-tiled BITCOS, 3 MoE)."""
     t = _abi.KwTile()
-    if not lib().ternocl_kw_tile_of(entry, BF16 if bf16 else FP16, M, N, K, E, ws_bytes, ctypes.byref(t)):
+    if not lib().ternocl_kw_tile_of(entry, M, N, K, E, ws_bytes, ctypes.byref(t)):
         return None
     return t.rows, t.cols, t.k_waves, t.k_slices, bool(t.repacked)
 

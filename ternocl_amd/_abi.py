@@ -29,7 +29,7 @@ SYMBOLS: dict[str, tuple] = {
     "ternocl_last_error": (C.c_char_p, []),
     "ternocl_version": (C.c_char_p, []),
     "ternocl_int2_gemm_ws_bytes": (Z, [I, I, I]),
-    "ternocl_kw_tile_of": (I, [I, I, I, I, I, I, Z, C.POINTER(KwTile)]),
+    "ternocl_kw_tile_of": (I, [I, I, I, I, I, Z, C.POINTER(KwTile)]),
     "ternocl_workspace_zero": (I, [P, Z, P]),
     "ternocl_int2_fp16_upcvt_gemm": (I, [I, P, P, P, P, P, P, I, I, I, I, I, P, Z, P]),
     "ternocl_int2_fp16_upcvt_gemm_ex": (I, [I, P, P, P, P, P, P, I, I, I, I, I, P, Z,

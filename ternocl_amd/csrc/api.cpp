@@ -69,7 +69,7 @@ size_t int2_gemm_ws_need(int M, int N, int K);
 ternocl_status int2_gemm_decode_run(int dtype, const uint32_t *B, uint32_t *D, int K, int N, hipStream_t st);
 // kernels (int2_gemm_kw.hip)
 size_t int2_gemm_kw_ws_need(int M, int N, int K);
-bool int2_gemm_kw_tile(int M, int N, int K, bool bf, size_t ws_bytes, bool force, ternocl_kw_tile &t);
+bool int2_gemm_kw_tile(int M, int N, int K, size_t ws_bytes, bool force, ternocl_kw_tile &t);
 bool int2_gemm_kw_run(int dtype, const void *A, const uint32_t *B, const void *S, void *C, const void *Other,
                       const void *Bias, int M, int N, int K, int postop, int out_f32, hipStream_t st, void *ws,
                       size_t ws_bytes, bool force, ternocl_status &s);
@@ -96,9 +96,9 @@ ternocl_status bitcos_gemm_mt_run(int dtype, const void *A, const uint32_t *Bc, 
                                   const void *Other, const void *Bias, int M, int N, int K, int postop,
                                   int out_f32, hipStream_t st);
 // kernels (bitcos_kw.hip): how a call of the M-tiled entry runs there (0: not)
-int bitcos_kw_auto(int M, int N, int K, bool bf, bool repack, const void *A, const void *Bc, const void *S, const void *C,
+int bitcos_kw_auto(int M, int N, int K, bool repack, const void *A, const void *Bc, const void *S, const void *C,
                    const void *Other, const void *Bias);
-bool bitcos_kw_tile(int M, int N, int K, bool bf, ternocl_kw_tile &t);
+bool bitcos_kw_tile(int M, int N, int K, ternocl_kw_tile &t);
 ternocl_status bitcos_kw_run(int dtype, const void *A, const uint32_t *Bc, const void *S, void *C, const void *Other,
                              const void *Bias, int M, int N, int K, int postop, int out_f32, hipStream_t st);
 ternocl_status bitcos_slice_ranks_run(const uint32_t *Bc, uint32_t *SR, int N, int K, int ls,
@@ -211,13 +211,13 @@ size_t ternocl_int2_gemm_ws_bytes(int M, int N, int K) {
     return a > b ? a : b;
 }
 
-int ternocl_kw_tile_of(int entry, int dtype, int M, int N, int K, int E, size_t ws_bytes, ternocl_kw_tile *tile) {
+int ternocl_kw_tile_of(int entry, int M, int N, int K, int E, size_t ws_bytes, ternocl_kw_tile *tile) {
     ternocl_kw_tile t = {0, 0, 0, 0, 0};
-    const bool bf = dtype == TERNOCL_BF16, ok = M >= 1 && N >= 16 && N % 16 == 0 && K >= kGS && K % kGS == 0;
+    const bool ok = M >= 1 && N >= 16 && N % 16 == 0 && K >= kGS && K % kGS == 0;
     bool kw = false;
-    if (ok && entry == 0) kw = int2_gemm_kw_tile(M, N, K, bf, ws_bytes, false, t);
+    if (ok && entry == 0) kw = int2_gemm_kw_tile(M, N, K, ws_bytes, false, t);
     else if (ok && entry == 1) kw = int2_int8_kw_tile(M, N, K, ws_bytes, t);
-    else if (ok && entry == 2) kw = bitcos_kw_tile(M, N, K, bf, t);
+    else if (ok && entry == 2) kw = bitcos_kw_tile(M, N, K, t);
     else if (ok && entry == 3 && E >= 1) kw = moe_kw_tile_of(M, E, N, K, t);
     if (tile) *tile = t;
     return kw ? 1 : 0;
@@ -459,7 +459,7 @@ ternocl_status ternocl_bitcos_fp16_upcvt_gemm_mt(int dtype, const void *A, const
     if (!ws) {  // the tiles decode the BITCOS weights themselves
         if ((size_t)M * K * 2 >= kMaxBufBytes)
             FAIL(TERNOCL_ERR_UNSUPPORTED_SHAPE, "the M-tiled BITCOS GEMM takes A below 2^31 bytes");
-        if (bitcos_kw_auto(M, N, K, dtype == TERNOCL_BF16, false, A, B, S, C, Other, Bias))
+        if (bitcos_kw_auto(M, N, K, false, A, B, S, C, Other, Bias))
             return bitcos_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream);
         return bitcos_gemm_mt_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream);
     }
@@ -470,7 +470,7 @@ ternocl_status ternocl_bitcos_fp16_upcvt_gemm_mt(int dtype, const void *A, const
         FAIL(TERNOCL_ERR_UNSUPPORTED_SHAPE, "the M-tiled BITCOS path takes A and the re-packed weights below 2^31 bytes");
     const hipStream_t st = (hipStream_t)stream;
     uint32_t *W2 = (uint32_t *)((uint8_t *)ws + kWsHeader);
-    const int kw = bitcos_kw_auto(M, N, K, dtype == TERNOCL_BF16, true, A, B, S, C, Other, Bias);
+    const int kw = bitcos_kw_auto(M, N, K, true, A, B, S, C, Other, Bias);
     if (kw == 1) return bitcos_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, st);
     if ((s = bitcos_to_int2_run(B, SR, ls, W2, N, K, st)) != TERNOCL_OK) return s;
     if (kw == 2 && int2_gemm_kw_run(dtype, A, W2, S, C, Other, Bias, M, N, K, postop, out_f32, st, nullptr, 0, true, s))

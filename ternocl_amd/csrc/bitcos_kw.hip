@@ -19,7 +19,7 @@
 
 namespace tcl {
 // (int2_gemm_kw.hip)
-void int2_gemm_kw_model(int M, int N, int K, bool bf, double &kw_us, double &other_us, int &wk, bool &square);
+void int2_gemm_kw_model(int M, int N, int K, double &kw_us, double &other_us, int &wk, bool &square);
 namespace {
 
 // BITCOS weights as the walk's B source (gemm_kw.hpp): per unit of 64 rows the
@@ -244,18 +244,18 @@ int bckw_tile(int M, int N, int K, int wk, double &us) {
     return best;
 }
 
-// The route of a call by (M, N, K, type) alone, the same with and without the
+// The route of a call by (M, N, K) alone, the same with and without the
 // re-pack workspace: a sum's bits depend on the waves over K only, so the two
 // calls agree bit for bit -- through these tiles, or the re-packed words on the
 // int2 engine's with as many waves over K, or (false) the 128-row tiles.  wk: the
 // waves over K; repacked: with a workspace the re-pack is ahead.
-bool bckw_route(int M, int N, int K, bool bf, int &wk, bool &repacked) {
+bool bckw_route(int M, int N, int K, int &wk, bool &repacked) {
     if (M <= 8 || M > 1024) return false;
     double direct, kw, other, chosen;
     int kwk;
     bool square;
     const int t = bckw_tile(M, N, K, 0, direct);
-    int2_gemm_kw_model(M, N, K, bf, kw, other, kwk, square);
+    int2_gemm_kw_model(M, N, K, kw, other, kwk, square);
     const double repack = 6.0 + 0.75 * K / 1024.0 + 5.5e-8 * K * N;  // k_bitcos_to_int2
     repacked = repack + kw < direct;
     wk = repacked ? kwk : kBcTiles[t].wk;
@@ -272,11 +272,11 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 // (for ternocl_kw_tile_of: the tile of an M-tiled call on aligned operands; repacked:
 // the workspace form runs int2_gemm_kw_run on the re-packed words)
-bool bitcos_kw_tile(int M, int N, int K, bool bf, ternocl_kw_tile &t) {
+bool bitcos_kw_tile(int M, int N, int K, ternocl_kw_tile &t) {
     int wk;
     bool repacked;
     double us;
-    if (!bckw_route(M, N, K, bf, wk, repacked)) return false;
+    if (!bckw_route(M, N, K, wk, repacked)) return false;
     const BcTile &b = kBcTiles[bckw_tile(M, N, K, wk, us)];
     t = {b.bm, b.bn, b.wk, 1, repacked};
     return true;
@@ -284,12 +284,12 @@ bool bitcos_kw_tile(int M, int N, int K, bool bf, ternocl_kw_tile &t) {
 
 // How a call of the M-tiled entry runs here: 0 not, 1 bitcos_kw_run, 2 (repack:
 // the caller re-packs the weights) int2_gemm_kw_run on the re-packed words.
-int bitcos_kw_auto(int M, int N, int K, bool bf, bool repack, const void *A, const void *Bc, const void *S, const void *C,
+int bitcos_kw_auto(int M, int N, int K, bool repack, const void *A, const void *Bc, const void *S, const void *C,
                    const void *Other, const void *Bias) {
     int wk;
     bool repacked;
     if (!aligned16(A) || !aligned16(Bc) || !aligned16(S) || !aligned16(C) || !aligned16(Other) || !aligned16(Bias) ||
-        !bckw_route(M, N, K, bf, wk, repacked))
+        !bckw_route(M, N, K, wk, repacked))
         return 0;
     return repack && repacked ? 2 : 1;
 }
@@ -300,7 +300,7 @@ ternocl_status bitcos_kw_run(int dtype, const void *A, const uint32_t *Bc, const
     int wk;
     bool repacked;
     double us;
-    bckw_route(M, N, K, bf, wk, repacked);
+    bckw_route(M, N, K, wk, repacked);
     auto go = [&](auto cfg) {
         typedef decltype(cfg) Cfg;
         return bf ? bckw_launch<Cfg, true>(A, Bc, S, C, Other, Bias, M, N, K, postop, out_f32, st)

@@ -119,7 +119,9 @@ struct KwPlan {
 
 // The cheapest tile and slice count by that model.  Further rounds cost their
 // K walk and half a base each (M = 300, K = 4096, N = 14336 on 64 x 64 tiles, 5
-// rounds: 64.9 modelled, 61.3 measured); a K split costs 1.2 us and its slice
+// rounds: 64.9 modelled, 61.3 measured), a whole base on the 128-column tiles of 64
+// rows and more, one workgroup a CU (M = 293, K = 6272, N = 22528 on 64 x 128, 4
+// rounds: 136 modelled, 140 measured); a K split costs 1.2 us and its slice
 // sums' round trip at 4 TB/s (M = 32, K = 14336, N = 4096 on 32 x 64 tiles, 4
 // slices: 13.6 modelled, 13.3 measured against 23.6 unsplit).
 KwPlan kw_plan(int M, int N, int K, bool split) {
@@ -131,7 +133,7 @@ KwPlan kw_plan(int M, int N, int K, bool split) {
         for (int ks = 1; ks <= 8; ++ks) {
             if (ks > 1 && (!split || K / ks < 512 || tiles * ks > 1024 || tiles * 16 > (long)kWsHeader)) break;
             const double rounds = (double)((tiles * ks + 255) / 256);
-            double us = t.base * (0.5 + 0.5 * rounds) + t.slope * rounds * K / (1024.0 * ks);
+            double us = t.base * (t.bm * t.bn > 4096 ? rounds : 0.5 + 0.5 * rounds) + t.slope * rounds * K / (1024.0 * ks);
             if (ks > 1) us += 1.2 + 8e-6 * ks * M * N / 4.0;
             if (us < best.us - 1e-9) best = {i, ks, us};
         }
@@ -141,21 +143,25 @@ KwPlan kw_plan(int M, int N, int K, bool split) {
 
 // The 128-row tile engine's time (int2_gemm_mfma.hip) by the same kind of fit, over its
 // plan: 128 x 128 tiles (M = 32 / 512 / 1024, K = N = 4096: 39.8 / 43.5 / 48.9
-// us), 128 x 256 tiles, dearer in bf16 (M = 300, K = 4096, N = 14336: 67.1; fp16 M = 194,
-// K = 13184, N = 23936: 183, M = 64, K = 5376, N = 21504: 53), 128 x 512 tiles (N =
-// 14336: 103) and their K split.  Both fits are
-// good to some 5%, so this engine is taken where it is ahead by more (kKwMargin).
+// us), 128 x 256 tiles (M = 1236, K = 4096, N = 6320: 66.8), 128 x 512 tiles (N =
+// 14336: 103; fewer than 192 of them, M = 1491, K = 9984, N = 5456: 193) and their K
+// split (M = 212, K = 9728, N = 13760: 81.7; M = 774, K = 10752, N = 3600: 88.4).  Both
+// fits are good to some 5%, so this engine is taken where it is ahead by more
+// (kKwMargin): of 18321 random calls of more than 16 rows, with and without the
+// workspace, none loses more than 3% (M to 2048, K to 14336, N to 34816).  With 24.5 k /
+// ks + 2e-6 ks M N for the split, and 128 x 256 tiles dearer in bf16, which they are
+// not, 65 did: the examples above took 81, 239, 91 and 99 us here.
 constexpr double kKwMargin = 0.95;
-double kw_other_us(int M, int N, int K, bool split, bool bf) {
+double kw_other_us(int M, int N, int K, bool split) {
     auto tiles = [&](int BM, int BN) { return (double)((long)((M + BM - 1) / BM) * ((N + BN - 1) / BN)); };
     const double k = K / 1024.0, wide = tiles(128, 512), half = tiles(128, 256), square = tiles(128, 128);
     if (wide >= 192) return 5.0 + 24.5 * k * (wide <= 256 ? 1.0 : wide / 256.0);
     const bool h = gemm_half_tile(M, N);
     const int ks = split && !(h && half >= 192) ? gemm_splits(M, N, K) : 1;
-    if (ks > 1) return 8.0 + 24.5 * k / ks + 8e-6 * ks * M * N / 4.0;
-    if (h) return 5.0 + (6.4 + 9.0 * half / 256.0 + (bf ? 3.0 : 0.0)) * k;
+    if (ks > 1) return 8.0 + 22.0 * k / ks * (wide * ks > 256 ? 2.0 : 1.0) + 1.4e-6 * ks * M * N;
+    if (h) return 7.1 + (9.9 + 5.6 * half / 256.0) * k;
     if (square <= 512) return 3.2 + (9.3 + 1.8 * std::min(square, 256.0) / 256.0) * k * (square > 256 ? 1.5 : 1.0);
-    return 5.0 + 24.5 * k * (wide <= 256 ? 1.0 : wide / 256.0);
+    return 5.0 + 22.0 * k;
 }
 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
@@ -165,45 +171,46 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 // The times the two models give a call without a K split (the M-tiled BITCOS
 // GEMM's choice, bitcos_kw.hip); wk: the waves over K of this engine's tile; square:
 // whether the other runs 128 x 128 tiles.
-void int2_gemm_kw_model(int M, int N, int K, bool bf, double &kw_us, double &other_us, int &wk, bool &square) {
+void int2_gemm_kw_model(int M, int N, int K, double &kw_us, double &other_us, int &wk, bool &square) {
     const KwPlan p = kw_plan(M, N, K, false);
     kw_us = p.us;
-    other_us = kw_other_us(M, N, K, false, bf);
+    other_us = kw_other_us(M, N, K, false);
     wk = p.tile <= 1 ? 8 : 4;
     square = gemm_tile_is_square(M, N);
 }
 
 // Whether plan p is the automatic engine of a call of M > 8 rows: always up to 16
-// rows (the MFMA GEMV is 2-3x its time there), above where its model is ahead of
+// rows (the MFMA GEMV is 2-3x its time there from K = 4096 on; with K <= 512 it is 2-20%
+// ahead, 0.2-0.9 us, but its sums are less exact), above where its model is ahead of
 // the 128-row tile engine's.  split: whether K slices may use a workspace.
-static bool kw_wins(const KwPlan &p, int M, int N, int K, bool split, bool bf) {
-    return M <= 16 || (M <= 2048 && p.us < kKwMargin * kw_other_us(M, N, K, split, bf));
+static bool kw_wins(const KwPlan &p, int M, int N, int K, bool split) {
+    return M <= 16 || (M <= 2048 && p.us < kKwMargin * kw_other_us(M, N, K, split));
 }
 
 // Workspace of the automatic plan's K split (0: none; none up to 16 rows).
 size_t int2_gemm_kw_ws_need(int M, int N, int K) {
     if (M <= 16 || M > 2048) return 0;
     const KwPlan p = kw_plan(M, N, K, true);
-    if (p.ks == 1 || !(kw_wins(p, M, N, K, true, false) || kw_wins(p, M, N, K, true, true))) return 0;
+    if (p.ks == 1 || !kw_wins(p, M, N, K, true)) return 0;
     return kWsHeader + (size_t)p.ks * M * N * 4;
 }
 
 // The tile and K slices of an automatic call on aligned operands with ws_bytes of
 // workspace (0: none), false where another engine runs it: the choice of
 // int2_gemm_kw_run, for ternocl_kw_tile_of.
-static bool kw_choose(int M, int N, int K, bool bf, size_t ws_bytes, bool force, KwPlan &p) {
+static bool kw_choose(int M, int N, int K, size_t ws_bytes, bool force, KwPlan &p) {
     bool split = ws_bytes > kWsHeader && M > 16;
     p = kw_plan(M, N, K, split);
     if (p.ks > 1 && ws_bytes < kWsHeader + (size_t)p.ks * M * N * 4) {
         p = kw_plan(M, N, K, false);
         split = false;
     }
-    return force || kw_wins(p, M, N, K, split, bf);
+    return force || kw_wins(p, M, N, K, split);
 }
 
-bool int2_gemm_kw_tile(int M, int N, int K, bool bf, size_t ws_bytes, bool force, ternocl_kw_tile &t) {
+bool int2_gemm_kw_tile(int M, int N, int K, size_t ws_bytes, bool force, ternocl_kw_tile &t) {
     KwPlan p;
-    if (M <= 8 || M > 2048 || !kw_choose(M, N, K, bf, ws_bytes, force, p)) return false;
+    if (M <= 8 || M > 2048 || !kw_choose(M, N, K, ws_bytes, force, p)) return false;
     t = {kKwTiles[p.tile].bm, kKwTiles[p.tile].bn, p.tile <= 1 ? 8 : 4, p.ks, 0};
     return true;
 }
@@ -220,7 +227,7 @@ bool int2_gemm_kw_run(int dtype, const void *A, const uint32_t *B, const void *S
         !aligned16(Bias))
         return false;
     KwPlan p;
-    if (!kw_choose(M, N, K, bf, ws && aligned16(ws) ? ws_bytes : 0, force, p)) return false;
+    if (!kw_choose(M, N, K, ws && aligned16(ws) ? ws_bytes : 0, force, p)) return false;
     uint64_t *cnt = p.ks > 1 ? (uint64_t *)ws : nullptr;
     float *part = p.ks > 1 ? (float *)((uint8_t *)ws + kWsHeader) : nullptr;
     auto go = [&](auto cfg) {

@@ -262,7 +262,7 @@ def test_k_slices_on_a_workspace_from_other_use(dev, M, K, N, fill):
 
     def call(entry, word):
         need = (T.int2_int8_gemm_ws_bytes if entry else T.int2_gemm_ws_bytes)(M, N, K)
-        assert T.kw_tile_of(entry, True, M, N, K, ws_bytes=need)[3] > 1, "no K slices"
+        assert T.kw_tile_of(entry, M, N, K, ws_bytes=need)[3] > 1, "no K slices"
         ws = torch.full((need // 4,), word, dtype=torch.int32, device="cuda")
         C = torch.zeros((M, N), dtype=A.dtype, device="cuda")
         if entry:

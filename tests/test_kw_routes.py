@@ -25,7 +25,7 @@ MOE = [
 def test_moe_engine(Tk, E, topk, H, I, taken):
     """The layer's products (N, K) = (I, H) and (H, I) take the same engine, whichever is faster."""
     import ternocl_amd as T
-    up, down = (T.kw_tile_of(3, True, Tk * topk, N, K, E) for N, K in ((I, H), (H, I)))
+    up, down = (T.kw_tile_of(3, Tk * topk, N, K, E) for N, K in ((I, H), (H, I)))
     assert (up is not None) == taken and (down is not None) == taken
 
 
@@ -45,6 +45,30 @@ BITCOS = [
 @pytest.mark.parametrize("M,K,N,tile", BITCOS)
 def test_bitcos_engine(M, K, N, tile):
     import ternocl_amd as T
-    for bf16 in (False, True):
-        got = T.kw_tile_of(2, bf16, M, N, K)
-        assert (got[:3] if got else None) == tile
+    got = T.kw_tile_of(2, M, N, K)
+    assert (got[:3] if got else None) == tile
+
+
+# (M, K, N, workspace, taken): the int2 GEMM on the MFMA GEMV (M <= 16) or the
+# 128-row tiles / here
+INT2 = [
+    (16, 512, 2256, False, True),       # the GEMV 4.4 / 4.7, but less exact sums
+    (16, 4096, 4096, False, True),      # 17 / 8.2
+    (212, 9728, 13760, True, False),    # four slices of 128 x 512 tiles: 81.7 / 91.2
+    (774, 10752, 3600, True, False),    # 88.4 / 98.7
+    (488, 10240, 5888, True, False),    # 81.0 / 90.2
+    (1236, 4096, 6320, False, False),   # 128 x 256 tiles: 66.8 / 81.4
+    (164, 2816, 32528, False, False),   # 51.9 / 55.8
+    (293, 6272, 22528, False, (32, 128)),  # 128 x 512 tiles 124.8; 64 x 128 tiles 140.1, 32 x 128 122.1
+    (1491, 9984, 5456, False, False),   # 193 / 239
+    (32, 14336, 4096, True, True),      # 131 / 13
+    (200, 5120, 5120, True, True),      # 50 / 25
+    (512, 4096, 4096, True, True),      # 43 / 24
+]
+
+
+@pytest.mark.parametrize("M,K,N,ws,taken", INT2)
+def test_int2_engine(M, K, N, ws, taken):
+    import ternocl_amd as T
+    got = T.kw_tile_of(0, M, N, K, ws_bytes=T.int2_gemm_ws_bytes(M, N, K) if ws else 0)
+    assert (got is not None) == bool(taken) and (taken in (False, True) or got[:2] == taken)
