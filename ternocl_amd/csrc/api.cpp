@@ -97,10 +97,10 @@ ternocl_status bitcos_gemm_mt_run(int dtype, const void *A, const uint32_t *Bc, 
                                   int out_f32, hipStream_t st);
 // kernels (bitcos_kw.hip): how a call of the M-tiled entry runs there (0: not)
 int bitcos_kw_auto(int M, int N, int K, bool repack, const void *A, const void *Bc, const void *S, const void *C,
-                   const void *Other, const void *Bias);
+                   const void *Other, const void *Bias, int &tile);
 bool bitcos_kw_tile(int M, int N, int K, ternocl_kw_tile &t);
 ternocl_status bitcos_kw_run(int dtype, const void *A, const uint32_t *Bc, const void *S, void *C, const void *Other,
-                             const void *Bias, int M, int N, int K, int postop, int out_f32, hipStream_t st);
+                             const void *Bias, int M, int N, int K, int postop, int out_f32, int tile, hipStream_t st);
 ternocl_status bitcos_slice_ranks_run(const uint32_t *Bc, uint32_t *SR, int N, int K, int ls,
                                       hipStream_t st);
 ternocl_status bitcos_dequant_run(int dtype, const uint32_t *Bc, const void *S, void *W, int N, int K,
@@ -459,8 +459,9 @@ ternocl_status ternocl_bitcos_fp16_upcvt_gemm_mt(int dtype, const void *A, const
     if (!ws) {  // the tiles decode the BITCOS weights themselves
         if ((size_t)M * K * 2 >= kMaxBufBytes)
             FAIL(TERNOCL_ERR_UNSUPPORTED_SHAPE, "the M-tiled BITCOS GEMM takes A below 2^31 bytes");
-        if (bitcos_kw_auto(M, N, K, false, A, B, S, C, Other, Bias))
-            return bitcos_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream);
+        int tile;
+        if (bitcos_kw_auto(M, N, K, false, A, B, S, C, Other, Bias, tile))
+            return bitcos_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, tile, (hipStream_t)stream);
         return bitcos_gemm_mt_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, (hipStream_t)stream);
     }
     const size_t need = ternocl_bitcos_gemm_mt_ws_bytes(K, N);
@@ -470,8 +471,9 @@ ternocl_status ternocl_bitcos_fp16_upcvt_gemm_mt(int dtype, const void *A, const
         FAIL(TERNOCL_ERR_UNSUPPORTED_SHAPE, "the M-tiled BITCOS path takes A and the re-packed weights below 2^31 bytes");
     const hipStream_t st = (hipStream_t)stream;
     uint32_t *W2 = (uint32_t *)((uint8_t *)ws + kWsHeader);
-    const int kw = bitcos_kw_auto(M, N, K, true, A, B, S, C, Other, Bias);
-    if (kw == 1) return bitcos_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, st);
+    int tile;
+    const int kw = bitcos_kw_auto(M, N, K, true, A, B, S, C, Other, Bias, tile);
+    if (kw == 1) return bitcos_kw_run(dtype, A, B, S, C, Other, Bias, M, N, K, postop, out_f32, tile, st);
     if ((s = bitcos_to_int2_run(B, SR, ls, W2, N, K, st)) != TERNOCL_OK) return s;
     if (kw == 2 && int2_gemm_kw_run(dtype, A, W2, S, C, Other, Bias, M, N, K, postop, out_f32, st, nullptr, 0, true, s))
         return s;

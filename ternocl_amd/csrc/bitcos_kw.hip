@@ -18,6 +18,7 @@
 #include <algorithm>
 
 namespace tcl {
+int bitcos_pick_ls(int N, int K);  // bitcos.hip
 // (int2_gemm_kw.hip)
 void int2_gemm_kw_model(int M, int N, int K, double &kw_us, double &other_us, int &wk, bool &square);
 namespace {
@@ -247,19 +248,23 @@ int bckw_tile(int M, int N, int K, int wk, double &us) {
 // The route of a call by (M, N, K) alone, the same with and without the
 // re-pack workspace: a sum's bits depend on the waves over K only, so the two
 // calls agree bit for bit -- through these tiles, or the re-packed words on the
-// int2 engine's with as many waves over K, or (false) the 128-row tiles.  wk: the
-// waves over K; repacked: with a workspace the re-pack is ahead.
-bool bckw_route(int M, int N, int K, int &wk, bool &repacked) {
+// int2 engine's with as many waves over K, or (false) the 128-row tiles.  tile: of
+// kBcTiles; repacked: with a workspace the re-pack is ahead.
+bool bckw_route(int M, int N, int K, int &tile, bool &repacked) {
     if (M <= 8 || M > 1024) return false;
     double direct, kw, other, chosen;
-    int kwk;
+    int kwk, wk;
     bool square;
     const int t = bckw_tile(M, N, K, 0, direct);
     int2_gemm_kw_model(M, N, K, kw, other, kwk, square);
-    const double repack = 6.0 + 0.75 * K / 1024.0 + 5.5e-8 * K * N;  // k_bitcos_to_int2
+    // k_bitcos_to_int2: a wave a slice walks its rows.  The slices are the caller's and bits
+    // must not depend on them: the library's own choice counts.  (5..95% of the sizes
+    // above within 0.88..1.09; without the slices 10 - 16 us were counted for 27 - 60 at K
+    // above ~5000 with few slices: M = 71 K = 10624 N = 4560 73.5 us against 40.4 direct.)
+    const double k = K / 1024.0, repack = 4.3 + 6.35 * k / bitcos_pick_ls(N, K) + 0.67 * k + 7.4e-8 * K * N;
     repacked = repack + kw < direct;
     wk = repacked ? kwk : kBcTiles[t].wk;
-    bckw_tile(M, N, K, wk, chosen);
+    tile = bckw_tile(M, N, K, wk, chosen);
     // ahead (by more than the fits' spread) of the re-pack and the 128-row tiles, and
     // without the workspace of the tiles that decode in place: 1.7 - 1.9x the int2 ones
     // on 128 x 128, 1.15 - 1.3x on the wider
@@ -273,41 +278,35 @@ bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 // (for ternocl_kw_tile_of: the tile of an M-tiled call on aligned operands; repacked:
 // the workspace form runs int2_gemm_kw_run on the re-packed words)
 bool bitcos_kw_tile(int M, int N, int K, ternocl_kw_tile &t) {
-    int wk;
+    int tile;
     bool repacked;
-    double us;
-    if (!bckw_route(M, N, K, wk, repacked)) return false;
-    const BcTile &b = kBcTiles[bckw_tile(M, N, K, wk, us)];
+    if (!bckw_route(M, N, K, tile, repacked)) return false;
+    const BcTile &b = kBcTiles[tile];
     t = {b.bm, b.bn, b.wk, 1, repacked};
     return true;
 }
 
-// How a call of the M-tiled entry runs here: 0 not, 1 bitcos_kw_run, 2 (repack:
-// the caller re-packs the weights) int2_gemm_kw_run on the re-packed words.
+// How a call of the M-tiled entry runs here: 0 not, 1 bitcos_kw_run on `tile`, 2
+// (repack: the caller re-packs the weights) int2_gemm_kw_run on the re-packed words.
 int bitcos_kw_auto(int M, int N, int K, bool repack, const void *A, const void *Bc, const void *S, const void *C,
-                   const void *Other, const void *Bias) {
-    int wk;
+                   const void *Other, const void *Bias, int &tile) {
     bool repacked;
     if (!aligned16(A) || !aligned16(Bc) || !aligned16(S) || !aligned16(C) || !aligned16(Other) || !aligned16(Bias) ||
-        !bckw_route(M, N, K, wk, repacked))
+        !bckw_route(M, N, K, tile, repacked))
         return 0;
     return repack && repacked ? 2 : 1;
 }
 
 ternocl_status bitcos_kw_run(int dtype, const void *A, const uint32_t *Bc, const void *S, void *C, const void *Other,
-                             const void *Bias, int M, int N, int K, int postop, int out_f32, hipStream_t st) {
+                             const void *Bias, int M, int N, int K, int postop, int out_f32, int tile, hipStream_t st) {
     const bool bf = dtype == TERNOCL_BF16;
-    int wk;
-    bool repacked;
-    double us;
-    bckw_route(M, N, K, wk, repacked);
     auto go = [&](auto cfg) {
         typedef decltype(cfg) Cfg;
         return bf ? bckw_launch<Cfg, true>(A, Bc, S, C, Other, Bias, M, N, K, postop, out_f32, st)
                   : bckw_launch<Cfg, false>(A, Bc, S, C, Other, Bias, M, N, K, postop, out_f32, st);
     };
     hipError_t e;
-    switch (bckw_tile(M, N, K, wk, us)) {
+    switch (tile) {
     case 0: e = go(KwCfg<1, 1, 1, 8, 4>{}); break;
     case 1: e = go(KwCfg<2, 1, 1, 8, 4>{}); break;
     case 2: e = go(KwCfg<2, 2, 1, 8, 4>{}); break;

@@ -38,7 +38,11 @@ BITCOS = [
     (10, 128, 33584, None),              # 32 x 32: 13.3 / 8.3 / 11.7
     (102, 640, 10432, None),             # 20.2 / 17.3 / 19.7
     (459, 768, 2400, None),              # 19.6 / 18.6 / 17.6
-    (32, 4096, 4096, (32, 32, 8)),       # 12.1 / 70 / 52
+    (32, 4096, 4096, (32, 32, 8)),       # 13.2 / 72 / 53
+    # the re-pack takes 27 - 60 us where K has few slices: it or the tiles that decode themselves
+    (71, 10624, 4560, (32, 32, 8, False)),    # 73.5 re-packed / 40.4
+    (366, 13696, 1488, (64, 64, 8, False)),   # 107.8 / 71.6
+    (64, 5376, 21504, (64, 64, 4, True)),     # 46.5 / 52.0
 ]
 
 
@@ -46,7 +50,7 @@ BITCOS = [
 def test_bitcos_engine(M, K, N, tile):
     import ternocl_amd as T
     got = T.kw_tile_of(2, M, N, K)
-    assert (got[:3] if got else None) == tile
+    assert (got and (got[:3] + got[4:])[:len(tile or ())]) == tile
 
 
 # (M, K, N, workspace, taken): the int2 GEMM on the MFMA GEMV (M <= 16) or the
