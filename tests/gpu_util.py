@@ -21,6 +21,18 @@ def dev_raw(a: np.ndarray, device="cuda:0"):
     return torch.from_numpy(a.view(view)).to(device)
 
 
+def off16(t):
+    """A copy of device tensor t that starts 4 bytes past a 16-byte boundary: the engines that load
+    16 bytes at a time leave such an operand to the tile engines."""
+    import torch
+    pad = 4 // t.element_size()
+    buf = torch.empty(t.numel() + pad, dtype=t.dtype, device=t.device)
+    out = buf[pad:].view(t.shape)
+    out.copy_(t)
+    assert out.data_ptr() % 16 == 4
+    return out
+
+
 def host_u16(t) -> np.ndarray:
     import torch
     return t.detach().view(torch.int16).cpu().numpy().view(np.uint16)

@@ -1,7 +1,8 @@
-"""GPU parity of the M-tiled BITCOS GEMM with K split over the waves (9 rows to a few hundred) at
-the edges of its tiles: 32- and 64-row tiles one row short, full and one row over, strips ending
-in one 16-column block, a K of one unit per wave and less, densities from empty sign streams to a
-sign a row; the call with the re-pack workspace gives the same bits as the one without.
+"""GPU parity of the M-tiled BITCOS GEMM with K split over the waves (9 rows to a few hundred) on
+every tile that it compiles, at the tiles' edges: one row short, full and one row over, strips
+ending in one 16-column block, a K of one unit per wave and less, densities from empty sign
+streams to a sign a row; the call with the re-pack workspace gives the same bits as the one
+without, also where the two run different kernels.
 
 fp32 outputs against float64 sums of the same factors: K exact products added in fp32 are within
 K 2^-24 sum|terms|."""
@@ -15,8 +16,22 @@ from tests.gpu_util import allclose_report, dev_dt, dev_raw, host_f32, host_u16
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(9, 128, 16), (31, 512, 2064), (33, 640, 1040), (64, 1408, 4112), (65, 5376, 272), (129, 768, 4112),
-          (200, 1024, 2064)]
+# (M, K, N): (rows, columns, waves over K, whether the workspace form re-packs) of the tile it runs
+# on, asserted (None: the 128-row tiles).  The re-packed words run on the int2 engine's tile of as
+# many waves over K, so the two forms' bits meet across two kernels there
+TILES = {
+    (9, 128, 16): None, (31, 512, 2064): (32, 32, 8, False), (33, 640, 1040): (32, 32, 8, False),
+    (65, 5376, 272): (32, 32, 8, False), (200, 1024, 2064): (32, 32, 8, False),
+    (33, 256, 4240): (64, 32, 8, False), (64, 1408, 4112): (64, 32, 8, False), (65, 384, 2832): (64, 32, 8, False),
+    (129, 1664, 3344): (64, 64, 8, False), (300, 1664, 1680): (64, 64, 8, False),
+    (65, 384, 5520): (64, 64, 4, False), (129, 768, 4112): (64, 64, 4, False),
+    (193, 4096, 4624): (32, 32, 8, True), (65, 896, 8208): (64, 64, 4, True),
+}
+
+
+def _on_tile(T, M, K, N, tile):
+    got = T.kw_tile_of(2, M, N, K)
+    assert (got and got[:3] + got[4:]) == tile, f"runs on {got}"
 
 
 def _run(T, torch, A, buf, S, other, bias_f, M, K, N, bf16, postop, out_f32, repack):
@@ -35,10 +50,11 @@ def _run(T, torch, A, buf, S, other, bias_f, M, K, N, bf16, postop, out_f32, rep
 
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("z", [0.0, 0.5, 1.0])
-@pytest.mark.parametrize("M,K,N", SHAPES)
+@pytest.mark.parametrize("M,K,N", TILES)
 def test_bitcos_kw_parity(dev, M, K, N, z, bf16):
     import torch
     import ternocl_amd as T
+    _on_tile(T, M, K, N, TILES[M, K, N])
     print(f"bitcos kw M={M} K={K} N={N} z={z} bf16={bf16}", flush=True)
     g = synth.rng(300 + M + K + N)
     A = synth.activations(g, (M, K), bf16)
@@ -60,10 +76,11 @@ def test_bitcos_kw_parity(dev, M, K, N, z, bf16):
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("postop", [0, 1, 2, 3, 4])
 @pytest.mark.parametrize("out_f32", [False, True])
-@pytest.mark.parametrize("M,K,N", [(20, 256, 1040), (100, 512, 4112)])
-def test_bitcos_kw_epilogues(dev, orc, M, K, N, bf16, postop, out_f32):
+@pytest.mark.parametrize("M,K,N,tile", [(20, 256, 1040, (32, 32, 8, False)), (100, 512, 4112, (64, 64, 4, False))])
+def test_bitcos_kw_epilogues(dev, orc, M, K, N, tile, bf16, postop, out_f32):
     import torch
     import ternocl_amd as T
+    _on_tile(T, M, K, N, tile)
     g = synth.rng(7 + postop + M)
     A = synth.activations(g, (M, K), bf16)
     buf, _ = synth.bitcos_weights(g, K, N, 0.4)

@@ -1,4 +1,5 @@
-"""GPU parity of the int2 prefill GEMM (M > 16; engine 3 at any M) through the C ABI.
+"""GPU parity of the int2 GEMM of more than 16 rows through the C ABI: on the automatic engine and
+on the tile engine (engine 3, at any M).
 
 Reference test design followed: int2_fp16_upcvt/validate.sh:8-10 (shape list
 with ragged M, fp16 + bf16), validate_epilogues.sh:19-36 (POSTOP 0..4 x DT /
@@ -24,14 +25,19 @@ SHAPES = [(17, 256, 48), (33, 1024, 272), (64, 4096, 4096), (100, 2048, 1040), (
           (77, 14336, 512), (2048, 2048, 16)]
 
 
+def _tile(T, engine):
+    return T.gemv_tile(T.GEMM) if engine == "tiles" else None
+
+
+@pytest.mark.parametrize("engine", ["auto", "tiles"])
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("M,K,N", SHAPES)
-def test_gemm_parity(dev, orc, M, K, N, bf16):
+def test_gemm_parity(dev, orc, M, K, N, bf16, engine):
     import torch
     import ternocl_amd as T
     print(f"gemm parity M={M} K={K} N={N} bf16={bf16}", flush=True)
     A, B, S, other, bias_f = int2_inputs(2000 + M + K + N, M, K, N, bf16)
-    dC, _ = int2_run(T, torch, A, B, S, other, bias_f, M, K, N, bf16, 0, False)
+    dC, _ = int2_run(T, torch, A, B, S, other, bias_f, M, K, N, bf16, 0, False, tile=_tile(T, engine))
     want, _ = int2_gold(orc, A, B, S, other, bias_f, M, K, N, bf16, 0, False)
     bad, dmax = allclose_report(formats.dt_to_f32(host_u16(dC), bf16), formats.dt_to_f32(want, bf16))
     assert bad == 0, f"{bad} elements outside 1e-3 + 1e-2*|ref| (max |d| {dmax})"
@@ -51,16 +57,17 @@ def test_gemm_engine_small_m(dev, orc, M):
     assert bad == 0, f"{bad} bad (max |d| {dmax})"
 
 
+@pytest.mark.parametrize("engine", ["auto", "tiles"])
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("postop", [0, 1, 2, 3, 4, 5])
 @pytest.mark.parametrize("out_f32", [False, True])
-def test_gemm_epilogues(dev, orc, bf16, postop, out_f32):
+def test_gemm_epilogues(dev, orc, bf16, postop, out_f32, engine):
     import torch
     import ternocl_amd as T
     M, K, N = 200, 1024, 528
     print(f"gemm epilogue bf16={bf16} postop={postop} f32={out_f32}", flush=True)
     A, B, S, other, bias_f = int2_inputs(70 + postop, M, K, N, bf16)
-    dC, _ = int2_run(T, torch, A, B, S, other, bias_f, M, K, N, bf16, postop, out_f32)
+    dC, _ = int2_run(T, torch, A, B, S, other, bias_f, M, K, N, bf16, postop, out_f32, tile=_tile(T, engine))
     want, _ = int2_gold(orc, A, B, S, other, bias_f, M, K, N, bf16, postop, out_f32)
     if out_f32:
         got, ref = host_f32(dC), want
@@ -70,25 +77,27 @@ def test_gemm_epilogues(dev, orc, bf16, postop, out_f32):
     assert bad == 0, f"{bad} bad (max |d| {dmax})"
 
 
+@pytest.mark.parametrize("engine", ["auto", "tiles"])
 @pytest.mark.parametrize("bf16", [False, True])
-def test_gemm_reference_distribution_rule(dev, orc, bf16):
+def test_gemm_reference_distribution_rule(dev, orc, bf16, engine):
     """The reference driver's own inputs (A ~ U[-5,5], S ~ U[0.75,15.75]) and
     pass rule (xetla_buff_cmp), at a prefill shape."""
     import torch
     import ternocl_amd as T
     M, K, N = 96, 5120, 1024
     A, B, S, other, bias_f = int2_inputs(98, M, K, N, bf16, ref_dist=True)
-    dC, _ = int2_run(T, torch, A, B, S, other, bias_f, M, K, N, bf16, 0, False)
+    dC, _ = int2_run(T, torch, A, B, S, other, bias_f, M, K, N, bf16, 0, False, tile=_tile(T, engine))
     want, _ = int2_gold(orc, A, B, S, other, bias_f, M, K, N, bf16, 0, False)
     assert xetla_cmp(host_u16(dC), want, bf16) == 0
 
 
-def test_gemm_deterministic(dev, orc):
+@pytest.mark.parametrize("engine", ["auto", "tiles"])
+def test_gemm_deterministic(dev, orc, engine):
     import torch
     import ternocl_amd as T
     M, K, N, bf16 = 333, 2048, 1040, False
     A, B, S, other, bias_f = int2_inputs(6, M, K, N, bf16)
-    outs = [host_u16(int2_run(T, torch, A, B, S, other, bias_f, M, K, N, bf16, 0, False)[0])
+    outs = [host_u16(int2_run(T, torch, A, B, S, other, bias_f, M, K, N, bf16, 0, False, tile=_tile(T, engine))[0])
             for _ in range(3)]
     assert all(np.array_equal(outs[0], o) for o in outs[1:]), "non-deterministic"
 

@@ -1,7 +1,7 @@
-"""GPU parity of the s8 x s2 GEMM with K split over the waves (5 rows to several hundred) at the
-edges of its tiles: 32- and 64-row tiles one row short, full and one row over, strips ending in
-one 16-column block, fewer groups than waves, and its K slices (a workspace); both quantization
-modes (the same bits), all four codes.
+"""GPU parity of the s8 x s2 GEMM with K split over the waves (5 rows to several hundred) on every
+tile that it compiles, at the tiles' edges: one row short, full and one row over, strips ending
+in one 16-column block, fewer groups than waves, with and without K slices (a workspace); both
+quantization modes (the same bits), all four codes.
 
 Gold: the int8 rows and scales of quant_a (bit-exact with the oracle, tests/test_gpu_int8.py) in
 float64.  The group dots are exact in int32; each of a column's G = K / 128 groups adds
@@ -17,9 +17,24 @@ from tests.gpu_util import allclose_report, dev_dt, dev_raw, host_f32, host_u16
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(5, 128, 16), (31, 256, 2064), (32, 1408, 4112), (33, 640, 1040), (63, 512, 8208), (65, 1152, 4112),
-          (129, 768, 2064), (200, 2048, 5136)]
-SPLIT = [(6, 14336, 1040), (48, 14336, 4096), (130, 8192, 528)]
+# (M, K, N): (rows, columns, waves over K, K slices) of the tile it runs on, asserted (None: the
+# tile engines)
+TILES = {
+    (5, 128, 16): None,  # (one group: the tile engine)
+    (7, 256, 1040): (32, 32, 8, 1), (31, 256, 2064): (32, 32, 8, 1), (32, 1408, 4112): (32, 32, 8, 1),
+    (33, 640, 1040): (32, 32, 8, 1),
+    (31, 384, 8208): (32, 64, 8, 1), (65, 1152, 4112): (32, 64, 8, 1), (129, 768, 2064): (32, 64, 8, 1),
+    (65, 640, 8208): (32, 64, 4, 1), (200, 2048, 5136): (32, 64, 4, 1),
+    (63, 512, 8208): (64, 64, 4, 1), (65, 512, 5520): (64, 64, 4, 1),
+    # K slices with the workspace
+    (6, 14336, 1040): (32, 32, 8, 7), (130, 8192, 528): (32, 32, 8, 3), (300, 8192, 272): (32, 64, 8, 5),
+    (65, 6144, 3088): (32, 64, 4, 3), (48, 14336, 4096): (64, 64, 4, 4),
+}
+
+
+def _on_tile(T, M, K, N, tile):
+    got = T.kw_tile_of(1, M, N, K, ws_bytes=T.int2_int8_gemm_ws_bytes(M, N, K))
+    assert (got and got[:4]) == tile, f"runs on {got}"
 
 
 def _case(T, torch, seed, M, K, N, bf16):
@@ -40,10 +55,11 @@ def _ws(T, torch, M, N, K):
 
 
 @pytest.mark.parametrize("bf16", [False, True])
-@pytest.mark.parametrize("M,K,N", SHAPES + SPLIT)
+@pytest.mark.parametrize("M,K,N", TILES)
 def test_int8_kw_parity(dev, M, K, N, bf16):
     import torch
     import ternocl_amd as T
+    _on_tile(T, M, K, N, TILES[M, K, N])
     print(f"int8 kw M={M} K={K} N={N} bf16={bf16} ws={T.int2_int8_gemm_ws_bytes(M, N, K)}", flush=True)
     B, SB, dA, dSA, dAq, dB, dSB = _case(T, torch, 900 + M + K + N, M, K, N, bf16)
     outs = []
@@ -71,12 +87,15 @@ def test_int8_kw_parity(dev, M, K, N, bf16):
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("postop", [1, 2, 3, 4, 5])
 @pytest.mark.parametrize("out_f32", [False, True])
-@pytest.mark.parametrize("M,K,N", [(7, 256, 1040), (40, 8192, 528), (100, 256, 2064)])
-def test_int8_kw_epilogues(dev, orc, M, K, N, bf16, postop, out_f32):
+@pytest.mark.parametrize("M,K,N,tile", [(7, 256, 1040, (32, 32, 8, 1)), (40, 8192, 528, (32, 32, 8, 7)),
+                                        (100, 384, 2064, (32, 64, 8, 1)), (65, 512, 5520, (64, 64, 4, 1)),
+                                        (100, 256, 2064, None)])
+def test_int8_kw_epilogues(dev, orc, M, K, N, tile, bf16, postop, out_f32):
     """Every epilogue on one and two columns per lane and after a K split, against the oracle's
     epilogue of the postop-0 fp32 sums (the same sums: the same plan)."""
     import torch
     import ternocl_amd as T
+    _on_tile(T, M, K, N, tile)
     _, _, _, dSA, dAq, dB, dSB = _case(T, torch, 40 + M, M, K, N, bf16)
     g = synth.rng(postop)
     other = synth.activations(g, (M, N), bf16)

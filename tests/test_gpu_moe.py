@@ -15,7 +15,7 @@ import numpy as np
 import pytest
 
 from ternocl_amd import formats, synth
-from tests.gpu_util import allclose_report, dev_dt, dev_raw, host_u16
+from tests.gpu_util import allclose_report, dev_dt, dev_raw, host_u16, off16
 
 pytestmark = pytest.mark.gpu
 
@@ -217,13 +217,15 @@ def test_moe_combine_rounding_special_values(dev, orc, bf16):
     assert np.isnan(gf[nan]).all() and np.array_equal(np.signbit(gf[nan]), np.signbit(Y[nan]))
 
 
-def _layer(T, torch, X, ids, RW, Tk, E, topk, H, I, W, bf16):
+def _layer(T, torch, X, ids, RW, Tk, E, topk, H, I, W, bf16, tiles=False):
+    """tiles: the packed weights off their 16-byte alignment, which only the 128-row tiles take (the
+    automatic engine otherwise)."""
     (Bg, Sg), (Bu, Su), (Bd, Sd) = W
+    dBg, dBu, dBd = (off16(dev_raw(B)) if tiles else dev_raw(B) for B in (Bg, Bu, Bd))
     dO = torch.zeros((Tk, H), dtype=torch.bfloat16 if bf16 else torch.float16, device="cuda")
     ws = torch.empty(T.int2_moe_prefill_ws_bytes(Tk, E, topk, H, I), dtype=torch.uint8, device="cuda")
     T.int2_moe_prefill(dev_dt(X, bf16), _ints(ids), dev_dt(RW, bf16), Tk, E, topk, H, I,
-                       dev_raw(Bg), dev_dt(Sg, bf16), dev_raw(Bu), dev_dt(Su, bf16), dev_raw(Bd),
-                       dev_dt(Sd, bf16), dO, ws)
+                       dBg, dev_dt(Sg, bf16), dBu, dev_dt(Su, bf16), dBd, dev_dt(Sd, bf16), dO, ws)
     torch.cuda.synchronize()
     return host_u16(dO)
 
@@ -250,8 +252,9 @@ def _weights(g, E, H, I, bf16):
     return _experts(g, E, H, I, bf16), _experts(g, E, H, I, bf16), _experts(g, E, I, H, bf16)
 
 
+@pytest.mark.parametrize("tiles", [False, True])
 @pytest.mark.parametrize("bf16", [False, True])
-def test_moe_layer_small(dev, orc, bf16):
+def test_moe_layer_small(dev, orc, bf16, tiles):
     import torch
     import ternocl_amd as T
     Tk, E, topk, H, I = 96, 8, 2, 256, 384
@@ -259,7 +262,7 @@ def test_moe_layer_small(dev, orc, bf16):
     X = synth.activations(g, (Tk, H), bf16)
     ids, RW = synth.moe_routing(g, Tk, E, topk, bf16)
     W = _weights(g, E, H, I, bf16)
-    got = formats.dt_to_f32(_layer(T, torch, X, ids, RW, Tk, E, topk, H, I, W, bf16), bf16)
+    got = formats.dt_to_f32(_layer(T, torch, X, ids, RW, Tk, E, topk, H, I, W, bf16, tiles), bf16)
     want = formats.dt_to_f32(_oracle_layer(orc, X, ids, RW, Tk, E, topk, H, I, W, bf16, T.moe_tile_rows()), bf16)
     bad, dmax = allclose_report(got, want)
     assert bad == 0, f"{bad} bad (max |d| {dmax})"
@@ -299,8 +302,9 @@ def test_moe_layer_multi_tile_experts(dev, orc, bf16):
 PAIR_COUNTS = [0, 64, 65, 1, 128, 129, 30, 200, 0, 63, 5, 7]
 
 
+@pytest.mark.parametrize("tiles", [False, True])
 @pytest.mark.parametrize("bf16", [False, True])
-def test_moe_layer_pair_tiles(dev, orc, bf16):
+def test_moe_layer_pair_tiles(dev, orc, bf16, tiles):
     """The layer's tile list (two experts' tails of at most 64 rows share a row tile, the
     others alone): every output within 1e-3 + 1e-2 |ref| of the oracle's stage composition,
     at a routing made for it (top-1, the rows per expert of PAIR_COUNTS, shuffled)."""
@@ -315,7 +319,7 @@ def test_moe_layer_pair_tiles(dev, orc, bf16):
     X = synth.activations(g, (Tk, H), bf16)
     RW = formats.f32_to_dt(np.ones(Tk, np.float32), bf16)
     W = _weights(g, E, H, I, bf16)
-    got = formats.dt_to_f32(_layer(T, torch, X, ids, RW, Tk, E, topk, H, I, W, bf16), bf16)
+    got = formats.dt_to_f32(_layer(T, torch, X, ids, RW, Tk, E, topk, H, I, W, bf16, tiles), bf16)
     want = formats.dt_to_f32(_oracle_layer(orc, X, ids, RW, Tk, E, topk, H, I, W, bf16, T.moe_tile_rows()), bf16)
     bad, dmax = allclose_report(got, want)
     assert bad == 0, f"{bad} of {got.size} outputs outside the rule (max |d| {dmax})"

@@ -1,5 +1,5 @@
 """GPU parity of the MoE prefill's grouped GEMMs for experts of few rows: empty experts, experts
-of 1, 31, 32, 33 and 64 rows, more than 64 experts (two steps of the tile search), dropped
+of 1, 31, 32, 33, 64 and 70 rows, more than 64 experts (two steps of the tile search), dropped
 assignments; the layer equals its stages bit for bit, and every output is within the rule of the
 oracle's stage composition (tests/test_gpu_moe.py)."""
 from __future__ import annotations
@@ -13,7 +13,7 @@ from tests.test_gpu_moe import _ints, _layer, _oracle_layer, _route, _weights
 
 pytestmark = pytest.mark.gpu
 
-# rows per expert (top-1): 32-row tiles, 64-row tiles (over 24 rows an expert), 70 experts
+# rows per expert (top-1): one 32-row tile, several, 70 experts
 COUNTS = [[0, 1, 31, 32, 33, 2, 0, 5, 64, 1, 1, 1], [40, 64, 65, 33, 0, 1, 63, 30],
           [1] * 30 + [0] * 10 + [3] * 29 + [70]]
 
@@ -29,6 +29,7 @@ def test_moe_kw_layer(dev, orc, counts, bf16):
     g.shuffle(ids)
     Tk = ids.size
     print(f"moe kw T={Tk} E={E} bf16={bf16}", flush=True)
+    assert T.kw_tile_of(3, Tk, I, H, E) and T.kw_tile_of(3, Tk, H, I, E), "another engine runs the layer"
     X = synth.activations(g, (Tk, H), bf16)
     RW = formats.f32_to_dt(np.ones(Tk, np.float32), bf16)
     W = _weights(g, E, H, I, bf16)
@@ -67,6 +68,7 @@ def test_moe_kw_dropped_ids(dev, orc):
     bad[::5] = np.where(np.arange(bad[::5].size) % 2 == 0, -1, E)
     rw0 = RW.copy()
     rw0[::5] = 0
+    assert T.kw_tile_of(3, Tk * topk, I, H, E) and T.kw_tile_of(3, Tk * topk, H, I, E)
     a = _layer(T, torch, X, bad, RW, Tk, E, topk, H, I, W, bf16)
     b = _layer(T, torch, X, ids, rw0, Tk, E, topk, H, I, W, bf16)
     assert np.array_equal(formats.dt_to_f32(a, bf16), formats.dt_to_f32(b, bf16))

@@ -139,9 +139,11 @@ def _bitcos_operands(T, torch, seed, K, N, z, bf16, ls):
     return dev_dt(A, bf16), dB, dev_dt(S, bf16), dSR
 
 
+@pytest.mark.parametrize("Mp", [32, 64, 300])
 @pytest.mark.parametrize("bf16", [False, True])
-def test_bitcos_mt_then_gemv_share_a_workspace(dev, bf16):
-    """The M-tiled BITCOS re-pack (after the header), then the split BITCOS GEMV."""
+def test_bitcos_mt_then_gemv_share_a_workspace(dev, bf16, Mp):
+    """An M-tiled BITCOS call (32 rows: decoded in place, the workspace unused; 64 and 300: the re-pack
+    after the header, then the K-over-waves GEMM / the 128-row tiles), then the split BITCOS GEMV."""
     import torch
     import ternocl_amd as T
     K, N = 5376, 21504
@@ -160,7 +162,8 @@ def test_bitcos_mt_then_gemv_share_a_workspace(dev, bf16):
         return host_u16(C)
     want = gemv(torch.zeros(need, dtype=torch.uint8, device="cuda"))
     ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
-    Mp = 64
+    tile = T.kw_tile_of(2, Mp, N, K)
+    assert (tile and tile[4]) == {32: False, 64: True, 300: None}[Mp]
     Ap = dev_dt(synth.activations(synth.rng(94), (Mp, K), bf16), bf16)
     Cp = torch.empty((Mp, N), dtype=dt, device="cuda")
     T.bitcos_fp16_upcvt_gemm_mt(Ap, B, S, SR, Cp, None, None, Mp, N, K, ls, ws)
