@@ -119,9 +119,7 @@ struct KwPlan {
 
 // The cheapest tile and slice count by that model.  Further rounds cost their
 // K walk and half a base each (M = 300, K = 4096, N = 14336 on 64 x 64 tiles, 5
-// rounds: 64.9 modelled, 61.3 measured), a whole base on the 128-column tiles of 64
-// rows and more, one workgroup a CU (M = 293, K = 6272, N = 22528 on 64 x 128, 4
-// rounds: 136 modelled, 140 measured); a K split costs 1.2 us and its slice
+// rounds: 64.9 modelled, 61.3 measured); a K split costs 1.2 us and its slice
 // sums' round trip at 4 TB/s (M = 32, K = 14336, N = 4096 on 32 x 64 tiles, 4
 // slices: 13.6 modelled, 13.3 measured against 23.6 unsplit).
 KwPlan kw_plan(int M, int N, int K, bool split) {
@@ -133,7 +131,7 @@ KwPlan kw_plan(int M, int N, int K, bool split) {
         for (int ks = 1; ks <= 8; ++ks) {
             if (ks > 1 && (!split || K / ks < 512 || tiles * ks > 1024 || tiles * 16 > (long)kWsHeader)) break;
             const double rounds = (double)((tiles * ks + 255) / 256);
-            double us = t.base * (t.bm * t.bn > 4096 ? rounds : 0.5 + 0.5 * rounds) + t.slope * rounds * K / (1024.0 * ks);
+            double us = t.base * (0.5 + 0.5 * rounds) + t.slope * rounds * K / (1024.0 * ks);
             if (ks > 1) us += 1.2 + 8e-6 * ks * M * N / 4.0;
             if (us < best.us - 1e-9) best = {i, ks, us};
         }
@@ -143,14 +141,15 @@ KwPlan kw_plan(int M, int N, int K, bool split) {
 
 // The 128-row tile engine's time (int2_gemm_mfma.hip) by the same kind of fit, over its
 // plan: 128 x 128 tiles (M = 32 / 512 / 1024, K = N = 4096: 39.8 / 43.5 / 48.9
-// us), 128 x 256 tiles (M = 1236, K = 4096, N = 6320: 66.8), 128 x 512 tiles (N =
-// 14336: 103; fewer than 192 of them, M = 1491, K = 9984, N = 5456: 193) and their K
-// split (M = 212, K = 9728, N = 13760: 81.7; M = 774, K = 10752, N = 3600: 88.4).  Both
-// fits are good to some 5%, so this engine is taken where it is ahead by more
-// (kKwMargin): of 18321 random calls of more than 16 rows, with and without the
-// workspace, none loses more than 3% (M to 2048, K to 14336, N to 34816).  With 24.5 k /
-// ks + 2e-6 ks M N for the split, and 128 x 256 tiles dearer in bf16, which they are
-// not, 65 did: the examples above took 81, 239, 91 and 99 us here.
+// us), 128 x 256 tiles (M = 1236, K = 4096, N = 6320: 68.2; M = 164, K = 2816, N = 32528:
+// 48.9), 128 x 512 tiles (N = 14336: 103; fewer than 192 of them, M = 1491, K = 9984, N =
+// 5456: 220) and their K split (M = 212, K = 9728, N = 13760: 81.7; M = 774, K = 10752, N =
+// 3600: 84.0).  Both fits are good to some 5%, so this engine is taken where it is
+// ahead by more (kKwMargin): of 7780 random calls with 5e9 multiply-adds or more (M to
+// 2048, K to 14336, N to 34816, both types, with and without the workspace, engines
+// timed in random order) 2 lose more than 3%, 45 with 24.5 k / ks + 2e-6 ks M N for the
+// split and 128 x 256 tiles dearer in bf16, which they are not: M = 164 took 53.2 us
+// here, M = 212 87.7, M = 774 91.2.
 constexpr double kKwMargin = 0.95;
 double kw_other_us(int M, int N, int K, bool split) {
     auto tiles = [&](int BM, int BN) { return (double)((long)((M + BM - 1) / BM) * ((N + BN - 1) / BN)); };

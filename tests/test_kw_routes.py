@@ -58,13 +58,13 @@ def test_bitcos_engine(M, K, N, tile):
 INT2 = [
     (16, 512, 2256, False, True),       # the GEMV 4.4 / 4.7, but less exact sums
     (16, 4096, 4096, False, True),      # 17 / 8.2
-    (212, 9728, 13760, True, False),    # four slices of 128 x 512 tiles: 81.7 / 91.2
-    (774, 10752, 3600, True, False),    # 88.4 / 98.7
-    (488, 10240, 5888, True, False),    # 81.0 / 90.2
-    (1236, 4096, 6320, False, False),   # 128 x 256 tiles: 66.8 / 81.4
-    (164, 2816, 32528, False, False),   # 51.9 / 55.8
-    (293, 6272, 22528, False, (32, 128)),  # 128 x 512 tiles 124.8; 64 x 128 tiles 140.1, 32 x 128 122.1
-    (1491, 9984, 5456, False, False),   # 193 / 239
+    (212, 9728, 13760, True, False),    # four slices of 128 x 512 tiles: 81.7 / 87.7
+    (774, 10752, 3600, True, False),    # 84.0 / 91.2
+    (488, 10240, 5888, True, False),    # 76.4 / 84.3
+    (1236, 10752, 2400, True, False),   # 79.6 / 87.3
+    (164, 2816, 32528, False, False),   # 128 x 256 tiles: 48.9 / 53.2
+    (293, 6272, 22528, False, True),    # 128 x 512 tiles: 136.7 / 122.8
+    (1004, 10240, 2576, False, True),   # 128 x 256 tiles: 99.3 / 81.3
     (32, 14336, 4096, True, True),      # 131 / 13
     (200, 5120, 5120, True, True),      # 50 / 25
     (512, 4096, 4096, True, True),      # 43 / 24
@@ -75,4 +75,4 @@ INT2 = [
 def test_int2_engine(M, K, N, ws, taken):
     import ternocl_amd as T
     got = T.kw_tile_of(0, M, N, K, ws_bytes=T.int2_gemm_ws_bytes(M, N, K) if ws else 0)
-    assert (got is not None) == bool(taken) and (taken in (False, True) or got[:2] == taken)
+    assert (got is not None) == taken
