@@ -240,10 +240,9 @@ __device__ __forceinline__ void kw_store(void *C, const uint16_t *Other, const v
     }
 }
 
-
-// A slice's arrival at its tile's counter (lane 0's atomics, broadcast): the
-// arrivals before this one.  Two 64-bit words, 0 between calls; the first counts
-// in steps of kKwStep.  A value that no count gives is left from another use of the
+// A slice's arrival at its tile's counter (lane 0's atomics, broadcast): whether it
+// is the last of ksn.  Two 64-bit words, 0 between calls; the first counts in steps
+// of kKwStep.  A value that no count gives is left from another use of the
 // workspace's memory (these calls' earlier engines took a workspace that nothing
 // had zeroed): every slice of the tile then sees one, and they count again in the
 // second word, by exchanges that take any value but a count of theirs for none.
@@ -251,29 +250,28 @@ __device__ __forceinline__ void kw_store(void *C, const uint16_t *Other, const v
 // counting by exchanges alone, retried whenever another slice arrives, took 4 us
 // more at 7 and 8 slices (M = 43 K = 7040 N = 512 9.0 -> 13.2).
 constexpr uint64_t kKwStep = 0x9E6D3A5171C3B20Full;
-__device__ __forceinline__ uint32_t kw_arrive(uint64_t *c, int ksn, int lane) {
-    uint32_t prev = 0;
+__device__ __forceinline__ bool kw_arrive(uint64_t *c, int ksn, int lane) {
+    bool last = false;
     if (lane == 0) {
         const uint64_t seen = __hip_atomic_fetch_add(c, kKwStep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        prev = ~0u;
-        for (int n = 0; n < ksn; ++n)
-            if (seen == (uint64_t)n * kKwStep) prev = (uint32_t)n;
-        if (prev == ~0u) {
+        last = seen == (uint64_t)(ksn - 1) * kKwStep;
+        bool count = last;
+        for (int n = 0; n < ksn - 1 && !count; ++n) count = seen == (uint64_t)n * kKwStep;
+        if (!count) {
             uint64_t e = 0;
-            while (true) {  // (fails only where another of the ksn slices arrived, or on the first guess)
-                prev = 0;
-                for (int n = 1; n < ksn; ++n)
-                    if (e == kKwStep + (uint64_t)n) prev = (uint32_t)n;
-                if (prev == (uint32_t)(ksn - 1)) break;
-                if (__hip_atomic_compare_exchange_strong(c + 1, &e, kKwStep + prev + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_AGENT))
-                    break;
-            }
-            if (prev == (uint32_t)(ksn - 1)) __hip_atomic_store(c + 1, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            uint32_t n;
+            do {  // (again only where another of the ksn slices arrived, or after the first guess)
+                n = 0;
+                for (int i = 1; i < ksn; ++i)
+                    if (e == kKwStep + (uint64_t)i) n = (uint32_t)i;
+                last = n == (uint32_t)(ksn - 1);
+            } while (!last && !__hip_atomic_compare_exchange_strong(c + 1, &e, kKwStep + n + 1, __ATOMIC_RELAXED,
+                                                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            if (last) __hip_atomic_store(c + 1, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        if (prev == (uint32_t)(ksn - 1)) __hip_atomic_store(c, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (last) __hip_atomic_store(c, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    return __builtin_amdgcn_readfirstlane(prev);
+    return __builtin_amdgcn_readfirstlane((uint32_t)last) != 0;
 }
 
 // The sums of the waves' K parts in wave order (through LDS, a round of row
@@ -385,11 +383,11 @@ __device__ __forceinline__ void kw_finish(f32x16_t acc[Cfg::MB][Cfg::CB], uint8_
     __syncthreads();  // every wave's sums are stored
     uint32_t *flag = (uint32_t *)lds;
     if (wave == 0) {
-        const uint32_t prev = kw_arrive(cnt, ksn, lane);
-        if (lane == 0) *flag = prev;
+        const bool last = kw_arrive(cnt, ksn, lane);
+        if (lane == 0) *flag = last;
     }
     __syncthreads();
-    if (*flag != (uint32_t)(ksn - 1)) return;  // (uniform)
+    if (!*flag) return;  // (uniform)
     for (int it = tid; it < Cfg::NRB * 256; it += Cfg::THREADS) {
         int r, n;
         rows_of(it, r, n);
