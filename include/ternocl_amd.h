@@ -79,23 +79,26 @@ const char *ternocl_version(void);
  * ws / ws_bytes: optional device scratch (16-byte aligned), kept from the XeTLA
  * plugin's entry (the acc/cnt buffers of its global k-slicing,
  * tools/xetla_epilogue_parity/parity.cpp:26-41); ternocl_int2_gemm_ws_bytes()
- * says how much a shape uses (0: pass NULL).  The prefill GEMM uses it for
- * deterministic split-K on shapes whose 128 x 512 tiles would leave CUs idle
- * (M = 1024, K = 14336, N = 4096: 4 K-slices): fp32 partial tiles per slice,
- * then a reduction that adds the slices in order and applies the epilogue,
- * the same bits on every run.  Without the scratch (NULL or short) those
- * shapes run on 128 x 128 tiles instead.  Shapes that run 192 to 256 tiles
- * of 128 x 256 (more than 256 tiles of 128 x 128: M = 1024, K = 4096,
- * N = 6144) take them with or without the scratch and leave it unused
- * (ternocl_int2_gemm_ws_bytes() still counts a split there: the sizes are
- * upper bounds).  The fp8 x fp4 GEMV splits K over
- * several workgroups per column strip where one workgroup per strip would
- * leave CUs idle or stage too much of A (K = 14336, N = 4096; M >= 3):
- * fp32 slice sums [slices][M][N] and a counter per 16-column strip, the
- * last workgroup of a strip adding the slices in order.  Its counters must
- * read zero before the first call on a scratch (ternocl_workspace_zero once);
- * every call leaves them zero.  Without the scratch the GEMV runs unsplit.
- * Calls that share one scratch must not overlap. */
+ * says how much a shape uses (0: pass NULL; none for M of 9..16).  Every use is
+ * a deterministic K split, fp32 slice sums added in slice order, the same bits
+ * on every run:
+ *   M > 16, the tile GEMM: shapes whose 128 x 512 tiles would leave CUs idle
+ *     (M = 1024, K = 14336, N = 4096: 4 slices), a reduction launch adding the
+ *     slices; without the scratch (NULL or short) the engine and tile that are
+ *     ahead unsplit.  Shapes that run 192 to 256 tiles of 128 x 256 (more than 256
+ *     tiles of 128 x 128: M = 1024, K = 4096, N = 6144) take them with or without
+ *     the scratch and leave it unused (ternocl_int2_gemm_ws_bytes() still counts a
+ *     split there: the sizes are upper bounds);
+ *   M > 16, the GEMM with K over the waves: few tiles of a long K (M = 48, K =
+ *     14336, N = 4096: 4 slices), a counter per tile electing the workgroup that
+ *     adds the slices; unsplit without the scratch.  Its counters take any
+ *     contents of the scratch;
+ *   M <= 8, the fp8 x fp4 GEMV: where one workgroup per column strip would leave
+ *     CUs idle or stage too much of A (K = 14336, N = 4096; M >= 3), a counter per
+ *     16-column strip; unsplit without the scratch.  Its counters must read zero
+ *     before the first call on a scratch (ternocl_workspace_zero once).
+ * Every call leaves its counters zero.  Calls that share one scratch must not
+ * overlap. */
 size_t ternocl_int2_gemm_ws_bytes(int M, int N, int K);
 ternocl_status ternocl_int2_fp16_upcvt_gemm(int dtype, const void *A, const uint32_t *B,
                                             const void *S, void *C, const void *Other,
@@ -106,7 +109,8 @@ ternocl_status ternocl_int2_fp16_upcvt_gemm(int dtype, const void *A, const uint
  * hardware.  Every field 0 = automatic. */
 typedef struct {
     int engine;          /* 1: VALU GEMV (v_dot2 MACs, M <= 8); 2: bf16/fp16 MFMA GEMV (M <= 16);
-                            3: MFMA prefill GEMM (any M, 128 x 128 tiles; the M > 16 engine);
+                            3: MFMA tile GEMM (any M; its tiles follow M and N; one of the
+                               automatic choices for M > 16);
                             4: block-scaled fp8 x fp4 MFMA GEMV (M <= 8, A 16-byte aligned;
                                the automatic choice where it applies);
                             5: its multi-strip form (M <= 8, K per slice <= 8192 and at
@@ -126,9 +130,10 @@ typedef struct {
 } ternocl_gemv_tile;
 
 /* Same as ternocl_int2_fp16_upcvt_gemm with an explicit tile (NULL = automatic:
- * the fp8 x fp4 GEMV for M <= 8 (A 16-byte aligned), the bf16/fp16 MFMA GEMV
- * for other M <= 16, the prefill GEMM above).  When M > 16 the engine
- * must be 0 or 3. */
+ * the fp8 x fp4 GEMV for M <= 8 (A 16-byte aligned), for other M the GEMM with
+ * K over the waves where operands are 16-byte aligned and, past 16 rows, it is
+ * ahead; otherwise the bf16/fp16 MFMA GEMV for M <= 16, the tile GEMM above).
+ * When M > 16 the engine must be 0 or 3. */
 ternocl_status ternocl_int2_fp16_upcvt_gemm_ex(int dtype, const void *A, const uint32_t *B,
                                                const void *S, void *C, const void *Other,
                                                const void *Bias, int M, int N, int K,
@@ -207,7 +212,8 @@ ternocl_status ternocl_quant_a(int dtype, const void *A, void *SA, int8_t *Aq, i
  * (QMODE 0), Aq and SA from ternocl_quant_a, A not read (may be NULL).
  * Aq NULL: in-GEMM mode (QMODE 1, :21-27, :61-99): the DT activations A are
  * quantized tile by tile with SA from ternocl_quant_a; the int8 values equal
- * quant_a's for every finite input, so both modes give identical C.
+ * quant_a's for every finite input, so both modes give identical C (A and Aq
+ * alike in being 16-byte aligned or not, which the engine depends on).
  * SB: DT [K/128, N]; B, C, Other, Bias, postop and out_f32 as
  * ternocl_int2_fp16_upcvt_gemm.  Any M >= 1; the A operand (M*K elements of
  * Aq or A) and B must each be below 2^31 bytes.  M <= 4 with N % 16 == 0 (Aq
@@ -228,10 +234,12 @@ ternocl_status ternocl_int2_int8_gemm(int dtype, const void *A, const int8_t *Aq
  * epilogue (shapes that run 128 x 256 tiles instead, M = 1024 K = 4096
  * N = 6144, leave the scratch unused).  The decode GEMV (M <= 4, both modes) splits long K (>= 8192)
  * over narrow N (< 6144 columns) the same way, a counter per 16-column strip
- * electing the workgroup that adds the slices in order.  Either way the same
- * bits on every run.  ws: ternocl_int2_int8_gemm_ws_bytes(M, N, K) bytes (0:
- * none used), 16-byte aligned, zeroed once before its first use (the GEMV's
- * counters return to zero by themselves; calls that share ws must not
+ * electing the workgroup that adds the slices in order, and so does the GEMM
+ * with K over the waves (M > 4, both modes) where it has few tiles of a long K, a
+ * counter per tile.  Each way the same bits on every run.  ws:
+ * ternocl_int2_int8_gemm_ws_bytes(M, N, K) bytes (0: none used), 16-byte
+ * aligned, zeroed once before its first use by the GEMV (the others take any
+ * contents; every call leaves its counters zero; calls that share ws must not
  * overlap); NULL or short: the call above. */
 size_t ternocl_int2_int8_gemm_ws_bytes(int M, int N, int K);
 ternocl_status ternocl_int2_int8_gemm_ws(int dtype, const void *A, const int8_t *Aq, const void *SA,

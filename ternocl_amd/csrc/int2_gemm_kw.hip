@@ -23,11 +23,15 @@
 //     b'), then a mask-and-set and a v_perm through the byte tables {0, s, 0,
 //     -s} (both DT types: exact +-s, three operations per pair).  Code 2 reads
 //     as 0.  CB adjacent columns per lane: one 4 CB-byte load per word row.
-//   * What bounds it: the traffic of the activations through L1 and LDS (each
-//     wave stores and reads every chunk of its rows once per 32 CB columns), not
-//     the weight stream: prefetching weights two or four units ahead measures
-//     the same, and a copy without the activation loads and stores takes half
-//     the time (M = 64, K = 5120, N = 34816: 50 -> 22-33 us over the tiles).
+//   * What bounds it: a wave's own instructions in a row, with one wave a SIMD (the
+//     64- and 128-column tiles) to cover them.  Counters: at M = 24, K = 4096, N =
+//     24576 (32 x 128) a wave issues VALU 51% of its time (the decode), waits 25%, the
+//     MFMAs are busy 24% and the LDS of a CU 15%; at M = 128, K = 4096, N = 14336 (64 x
+//     128) 41, 24, 34 and 21%; at M = 24, K = N = 4096 (32 x 32, two waves a SIMD) it
+//     waits 55%, for the first loads and the sums.  Not the weight stream: two or
+//     four units of weights ahead measure the same.  The activations' way through L1
+//     and LDS adds to all of it: a copy without their loads and stores takes half
+//     the time at M = 64, K = 5120, N = 34816 (50 -> 22-33 us over the tiles).
 //     Storing unit u itself at its start, on the critical path: 24 -> 21.7 us
 //     with the two buffers (M = 128, K = 4096, N = 14336).
 // Measured against the engines these calls took before (graph-timed, bf16,
